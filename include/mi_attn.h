@@ -62,7 +62,7 @@
 extern "C" {
 #endif
 
-#define MI_ATTN_ABI_VERSION 10
+#define MI_ATTN_ABI_VERSION 11
 
 #if defined(__GNUC__)
 #define MI_API __attribute__((visibility("default")))
@@ -343,6 +343,21 @@ MI_API int mi_attn_decode(const void* q, const void* k_new, const void* v_new,
                           const void* k_cache, const void* v_cache, const long long* cache_pos,
                           const float* gate, void* out, float* lse, float* workspace,
                           const mi_decode_shape* s, hipStream_t stream);
+
+/* Commit of a windowed step (window > 0; nanolab/mixers.py:435-450): of the
+ * rows [cache | new] those at positions < sinks or >= start + T - (window -
+ * sinks - 1) stay, in their order. mi_attn_cache_plan writes the kept rows'
+ * indices to `rows` (int32, cached + T), their positions to `positions`
+ * (int64, cached + T) and how many there are to `count` (int32; device memory
+ * or pinned host memory, readable once the call's work on `stream` is done). */
+MI_API int mi_attn_cache_plan(const long long* cache_pos, const mi_decode_shape* s, int* rows,
+                              long long* positions, int* count, hipStream_t stream);
+
+/* Copies the first `n` planned rows (n = the plan's count) of K and V to k_out
+ * and v_out, [B, Hkv, n, D] contiguous, 16-byte aligned, outside the cache. */
+MI_API int mi_attn_cache_gather(const void* k_new, const void* v_new, const void* k_cache,
+                                const void* v_cache, const int* rows, int n, void* k_out,
+                                void* v_out, const mi_decode_shape* s, hipStream_t stream);
 
 /* The K extent mi_mfma_probe expects for `dtype` (16 or 2), or -1. */
 MI_API int mi_mfma_probe_k(int dtype);

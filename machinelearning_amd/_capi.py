@@ -12,7 +12,7 @@ import ctypes
 import pathlib
 
 LIB_PATH = pathlib.Path(__file__).resolve().parent / "libmi_attn.so"
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 MI_F32, MI_F16, MI_BF16 = 0, 1, 2
 
@@ -99,6 +99,8 @@ SIGNATURES = {
     "mi_qk_prologue_bwd": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _PSHAPE, _P]),
     "mi_attn_decode_workspace": (ctypes.c_int, [_DSHAPE, ctypes.POINTER(ctypes.c_longlong)]),
     "mi_attn_decode": (ctypes.c_int, [_P] * 10 + [_DSHAPE, _P]),
+    "mi_attn_cache_plan": (ctypes.c_int, [_P, _DSHAPE, _P, _P, _P, _P]),
+    "mi_attn_cache_gather": (ctypes.c_int, [_P] * 5 + [ctypes.c_int, _P, _P, _DSHAPE, _P]),
     "mi_mfma_probe": (ctypes.c_int, [_P, _P, _P, ctypes.c_int, _P]),
     "mi_mfma_probe_k": (ctypes.c_int, [ctypes.c_int]),
     "mi_attn_error_string": (ctypes.c_char_p, [ctypes.c_int]),

@@ -137,6 +137,15 @@ struct DecParams {
   const float* gate;     // [B, T, H] output gate logits (nullptr: none)
 };
 
+// Parameters of a window cache's commit (cache_commit.hip): byte strides.
+struct CommitParams {
+  int B, T, Hkv, Lc;     // batch, new rows, kv heads, cached rows
+  int n;                 // rows kept per head
+  int chunks;            // 16-byte chunks per row
+  long long total;       // 2 * B * Hkv * n * chunks threads
+  long long k_sb, k_sh, v_sb, v_sh;   // cache batch / head strides in bytes
+};
+
 // Parameters of the fused q / k prologue (RMSNorm + RoPE, qk_prologue.hip).
 struct ProParams {
   int rows;        // B * T * H

@@ -49,6 +49,12 @@ hipError_t launch_decode(int dtype, const void* q, const void* kc, const void* v
                          const void* vn, void* out, float* lse, float* ws, const DecParams& p,
                          hipStream_t st);
 long long decode_workspace_floats(int dtype, const DecParams& p);
+hipError_t launch_cache_plan(const long long* pos, int Lc, int T, long long start, long long lo,
+                             long long sinks, int* rows, long long* pos_out, int* count,
+                             hipStream_t st);
+hipError_t launch_cache_gather(const void* kc, const void* vc, const void* kn, const void* vn,
+                               const int* rows, void* ko, void* vo, const CommitParams& p,
+                               hipStream_t st);
 hipError_t launch_prologue_fwd(int dtype_in, int dtype_out, int D, const void* x, const float* w,
                                const float* cs, const float* sn, void* out, float* rstd,
                                const ProParams& p, hipStream_t st);
@@ -677,6 +683,50 @@ int mi_attn_decode(const void* q, const void* k_new, const void* v_new, const vo
   p.gate = gate;
   return status_of(mi::launch_decode(s->dtype, q, k_cache, v_cache, k_new, v_new, out, lse,
                                      workspace, p, stream));
+}
+
+int mi_attn_cache_plan(const long long* cache_pos, const mi_decode_shape* s, int* rows,
+                       long long* positions, int* count, hipStream_t stream) {
+  const int st = validate_dec(s);
+  if (st) return st;
+  if (s->window <= 0) return MI_ERR_WINDOW;
+  if (!rows || !positions || !count) return MI_ERR_NULL;
+  const long long end = (long long)s->start + s->T;
+  return status_of(mi::launch_cache_plan(cache_pos, s->cached, s->T, s->start,
+                                         end - (s->window - s->sinks - 1), s->sinks, rows,
+                                         positions, count, stream));
+}
+
+int mi_attn_cache_gather(const void* k_new, const void* v_new, const void* k_cache,
+                         const void* v_cache, const int* rows, int n, void* k_out, void* v_out,
+                         const mi_decode_shape* s, hipStream_t stream) {
+  const int st = validate_dec(s);
+  if (st) return st;
+  if (n < 0 || n > (long long)s->cached + s->T) return MI_ERR_SHAPE;
+  const long long elem = s->dtype == MI_F32 ? 4 : 2;
+  mi::CommitParams p;
+  p.B = s->B;
+  p.T = s->T;
+  p.Hkv = s->Hkv;
+  p.Lc = s->cached;
+  p.n = n;
+  p.chunks = (int)(s->D * elem / 16);
+  p.total = 2LL * s->B * s->Hkv * n * p.chunks;
+  if (p.total == 0) return MI_OK;
+  if ((p.total + 255) / 256 > 0x7fffffffLL) return MI_ERR_SIZE;
+  p.k_sb = s->k_batch_stride * elem;
+  p.k_sh = s->k_head_stride * elem;
+  p.v_sb = s->v_batch_stride * elem;
+  p.v_sh = s->v_head_stride * elem;
+  if (!rows || !k_out || !v_out || (s->T > 0 && (!k_new || !v_new)) ||
+      (s->cached > 0 && (!k_cache || !v_cache)))
+    return MI_ERR_NULL;
+  if (!aligned16(k_out) || !aligned16(v_out) || (k_new && !aligned16(k_new)) ||
+      (v_new && !aligned16(v_new)) || (k_cache && !aligned16(k_cache)) ||
+      (v_cache && !aligned16(v_cache)))
+    return MI_ERR_ALIGN;
+  return status_of(mi::launch_cache_gather(k_cache, v_cache, k_new, v_new, rows, k_out, v_out, p,
+                                           stream));
 }
 
 int mi_mfma_probe_k(int dtype) {

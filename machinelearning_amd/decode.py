@@ -135,6 +135,58 @@ def _commit_append(cache, key, bufkey, old, new_rows, Lc, T):
     cache[key] = buf[:, :, :Lc + T]
 
 
+class _WindowCommit:
+    """The commit of a windowed step: which rows of [cache | block] stay, listed on
+    the GPU (``mi_attn_cache_plan``), and their copy into a new cache
+    (``mi_attn_cache_gather``).
+
+    How many rows stay depends on the cached positions, which live on the GPU, so
+    the host reads one count per step. The plan is launched before the step itself
+    and its count written to pinned memory: the wait is for the plan only, under
+    the step. Without ``pos`` (nothing evicted yet) the count follows from the
+    lengths, and nothing is waited for.
+    """
+
+    def __init__(self, lib, shp, cpos, Lc, T, start, window, sinks, dev, stream):
+        n = Lc + T
+        self.rows = torch.empty(n + 1, dtype=torch.int32, device=dev)
+        self.pos = torch.empty(n, dtype=torch.int64, device=dev)
+        if cpos is None:
+            end, lead = start + T, min(sinks, start + T)
+            self.known = lead + end - max(lead, end - (window - sinks - 1), 0)
+            self.count, self.done = self.rows[n:], None
+        else:
+            self.known = None
+            self.count = torch.empty(1, dtype=torch.int32, pin_memory=True)
+            self.done = torch.cuda.Event()
+        _capi.check(lib.mi_attn_cache_plan(None if cpos is None else cpos.data_ptr(),
+                                           ctypes.byref(shp), self.rows.data_ptr(),
+                                           self.pos.data_ptr(), self.count.data_ptr(), stream))
+        if self.done is not None:
+            self.done.record()
+
+    def wait(self) -> int:
+        """Rows that stay. (Also called when the step fails: the pinned count must
+        outlive the plan that writes it.)"""
+        if self.known is None:
+            self.done.synchronize()
+            self.known = int(self.count[0])
+        return self.known
+
+    def store(self, lib, shp, cache, k, v, ck, cv, stream, end):
+        n = self.wait()
+        B, _, Hkv, D = k.shape
+        nk = torch.empty(B, Hkv, n, D, dtype=k.dtype, device=k.device)
+        nv = torch.empty_like(nk)
+        _capi.check(lib.mi_attn_cache_gather(
+            k.data_ptr(), v.data_ptr(), None if ck is None else ck.data_ptr(),
+            None if cv is None else cv.data_ptr(), self.rows.data_ptr(), n, nk.data_ptr(),
+            nv.data_ptr(), ctypes.byref(shp), stream))
+        cache["k"], cache["v"] = nk, nv
+        cache["pos"] = self.pos[:n]
+        cache["end"] = end
+
+
 def attn_cached(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache: dict, commit: bool,
                 causal: bool = False, *, window: int = 0, sinks: int = 0,
                 scale: float | None = None, gate: torch.Tensor | None = None,
@@ -241,30 +293,23 @@ def attn_cached(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache: dict, 
 
     with _fc._on_device(q):
         stream = _fc._stream(q)
+        kept = (_WindowCommit(lib, shp, cpos, Lc, T, start, window, sinks, dev, stream)
+                if commit and window else None)
         ws = _workspace(dev, stream, nws) if nws > 0 else None
         st = lib.mi_attn_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), ptr(ck), ptr(cv),
                                 ptr(cpos), ptr(g), out.data_ptr(), ptr(lse), ptr(ws),
                                 ctypes.byref(shp), stream)
+        if kept is not None:
+            if st:
+                kept.wait()
+            else:
+                # Keep the sinks plus the tail the next block can still reach
+                # (mixers.py:437-448).
+                kept.store(lib, shp, cache, k, v, ck, cv, stream, start + T)
     _capi.check(st)
 
-    if commit:
+    if commit and not window:
         kt, vt = k.transpose(1, 2), v.transpose(1, 2)          # (B, Hkv, T, D) views
-        if window:
-            # Keep the sinks plus the tail the next block can still reach
-            # (mixers.py:437-448): positions < sinks or >= end - (w - s - 1).
-            end = start + T
-            tail = window - sinks - 1
-            apos = torch.arange(start, end, device=dev, dtype=torch.int64)
-            kpos = apos if Lc == 0 else torch.cat(
-                [cpos if cpos is not None else torch.arange(start, device=dev), apos])
-            live = (kpos < sinks) | (kpos >= end - tail)
-            k_full = kt if Lc == 0 else torch.cat([ck, kt], dim=2)
-            v_full = vt if Lc == 0 else torch.cat([cv, vt], dim=2)
-            cache["k"] = k_full[:, :, live].detach()
-            cache["v"] = v_full[:, :, live].detach()
-            cache["pos"] = kpos[live]
-            cache["end"] = end
-        else:
-            _commit_append(cache, "k", _KBUF, ck, kt, Lc, T)
-            _commit_append(cache, "v", _VBUF, cv, vt, Lc, T)
+        _commit_append(cache, "k", _KBUF, ck, kt, Lc, T)
+        _commit_append(cache, "v", _VBUF, cv, vt, Lc, T)
     return (out, lse) if return_lse else out

@@ -507,3 +507,40 @@ def test_decode_random_sweep(case):
     _step(q, k, v, cache, dtype, causal, window=window, sinks=sinks, gate=gt,
           tag=f"decode sweep d{i}: B{B} T{T} L{Lc} H{H}/{Hkv} D{D} {dtype} causal={causal} "
               f"w={window} s={sinks} gate={gate}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d).replace("torch.", ""))
+@pytest.mark.parametrize("Lc,T,window,sinks,evicted", [
+    (0, 1, 4, 1, False), (0, 9, 1, 0, False), (3, 2, 64, 4, False), (254, 1, 300, 4, False),
+    (62, 1, 64, 4, True), (255, 2, 256, 0, True), (255, 1, 2, 1, True), (513, 40, 300, 17, True),
+    (31, 3, 1, 0, True)])
+def test_window_commit_equals_boolean_indexing(dtype, Lc, T, window, sinks, evicted):
+    """The committed window cache == the live rows of cat([cache, block]) by boolean
+    indexing (mixers.py:437-448), whole values: row counts around the plan's 256-row
+    chunks, nothing left (window 1), positions in no order, a strided cache view."""
+    from machinelearning_amd.decode import attn_cached
+    g = torch.Generator(device="cuda").manual_seed(Lc * 7 + T)
+    B, H, Hkv, D = 2, 4, 2, 32
+
+    def rnd(*s):
+        return torch.randn(*s, device="cuda", generator=g).to(dtype)
+    q, k, v = rnd(B, T, H, D), rnd(B, T, Hkv, D), rnd(B, T, Hkv, D)
+    cache, start = {}, Lc
+    if Lc:
+        buf = rnd(2, B, Hkv, Lc + 5, D)
+        cache = {"k": buf[0, :, :, :Lc], "v": buf[1, :, :, :Lc]}
+    if evicted:
+        start = Lc + 40
+        cache["pos"] = torch.randperm(start, generator=g, device="cuda")[:Lc]
+    cache["end"] = start
+    kpos = torch.arange(start, start + T, device="cuda")
+    kf, vf = k.transpose(1, 2), v.transpose(1, 2)
+    if Lc:
+        kpos = torch.cat([cache.get("pos", torch.arange(Lc, device="cuda")), kpos])
+        kf, vf = torch.cat([cache["k"], kf], 2), torch.cat([cache["v"], vf], 2)
+    live = (kpos < sinks) | (kpos >= start + T - (window - sinks - 1))
+    with torch.no_grad():
+        attn_cached(q, k, v, cache, True, True, window=window, sinks=sinks)
+    assert torch.equal(cache["pos"], kpos[live]) and cache["end"] == start + T
+    assert torch.equal(cache["k"], kf[:, :, live]) and torch.equal(cache["v"], vf[:, :, live])
