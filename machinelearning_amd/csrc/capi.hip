@@ -31,6 +31,15 @@ hipError_t launch_bwd16_dkdv(int dtype, int D, const void* q, const void* k, con
 hipError_t launch_bwd16_dq(int dtype, int D, const void* q, const void* k, const void* v,
                            const void* dout, const float* lse, const float* delta, void* dq,
                            const AttnParams& p, hipStream_t st);
+bool f32_split_walk(const AttnParams& p, int heads, bool backward);
+hipError_t launch_f32_fwd(int D, const void* q, const void* k, const void* v, void* o, float* lse,
+                          const AttnParams& p, hipStream_t st);
+hipError_t launch_f32_dq(int D, const void* q, const void* k, const void* v, const void* dout,
+                         const float* lse, const float* delta, void* dq, const AttnParams& p,
+                         hipStream_t st);
+hipError_t launch_f32_dkdv(int D, const void* q, const void* k, const void* v, const void* dout,
+                           const float* lse, const float* delta, void* dk, void* dv,
+                           const AttnParams& p, hipStream_t st);
 hipError_t launch_sink_fwd(int dtype, int D, const void* q, const void* k, const void* v, void* o,
                            float* lse, const AttnParams& p, hipStream_t st);
 hipError_t launch_sink_dq(int dtype, int D, const void* q, const void* k, const void* v,
@@ -257,9 +266,10 @@ int run_fwd(const void* q, const void* k, const void* v, const float* gate, void
   mi::AttnParams p = params(s);
   p.gate = gate;
   p.o_res = o_res;
-  const hipError_t e = s->dtype == MI_F32
-                           ? mi::launch_fwd(s->dtype, s->D, q, k, v, o, lse, p, stream)
-                           : mi::launch_fwd16(s->dtype, s->D, q, k, v, o, lse, p, stream);
+  const hipError_t e =
+      s->dtype != MI_F32 ? mi::launch_fwd16(s->dtype, s->D, q, k, v, o, lse, p, stream)
+      : mi::f32_split_walk(p, s->H, false) ? mi::launch_f32_fwd(s->D, q, k, v, o, lse, p, stream)
+                                          : mi::launch_fwd(s->dtype, s->D, q, k, v, o, lse, p, stream);
   if (e != hipSuccess) return MI_ERR_LAUNCH;
   return status_of(mi::launch_sink_fwd(s->dtype, s->D, q, k, v, o, lse, p, stream));
 }
@@ -337,16 +347,18 @@ int run_dkdv(const void* q, const void* k, const void* v, const void* dout, cons
     p.kv_part = const_cast<float*>(delta) + split_offset(s);
   }
   const hipError_t e =
-      s->dtype == MI_F32
-          ? mi::launch_bwd_dkdv(s->dtype, s->D, q, k, v, dout, lse, delta, dk, dv, p, stream)
-          : mi::launch_bwd16_dkdv(s->dtype, s->D, q, k, v, dout, lse, delta, dk, dv, p, stream);
+      s->dtype != MI_F32
+          ? mi::launch_bwd16_dkdv(s->dtype, s->D, q, k, v, dout, lse, delta, dk, dv, p, stream)
+      : mi::f32_split_walk(p, s->Hkv, true)
+          ? mi::launch_f32_dkdv(s->D, q, k, v, dout, lse, delta, dk, dv, p, stream)
+          : mi::launch_bwd_dkdv(s->dtype, s->D, q, k, v, dout, lse, delta, dk, dv, p, stream);
   if (e != hipSuccess) return MI_ERR_LAUNCH;
   if (sp == SinkPass::kNone) return MI_OK;
   return status_of(mi::launch_sink_dkv(s->dtype, s->D, q, k, v, dout, lse, delta,
                                        sink_part(delta, s), dk, dv, nullptr, p, stream));
 }
 
-// With `o` set (16-bit inputs only), the dQ kernel also computes the delta
+// With `o` set (16-bit inputs, or float32 on the split-walk kernels), the dQ kernel also computes the delta
 // pass and writes both workspace planes (`delta`), from o and dlse.
 int run_dq(const void* q, const void* k, const void* v, const void* dout, const float* lse,
            const float* delta, void* dq, const mi_attn_shape* s, hipStream_t stream,
@@ -364,9 +376,11 @@ int run_dq(const void* q, const void* k, const void* v, const void* dout, const 
     p.o_res = const_cast<void*>(o_res);
   }
   const hipError_t e =
-      s->dtype == MI_F32
-          ? mi::launch_bwd_dq(s->dtype, s->D, q, k, v, dout, lse, delta, dq, p, stream)
-          : mi::launch_bwd16_dq(s->dtype, s->D, q, k, v, dout, lse, delta, dq, p, stream);
+      s->dtype != MI_F32
+          ? mi::launch_bwd16_dq(s->dtype, s->D, q, k, v, dout, lse, delta, dq, p, stream)
+      : mi::f32_split_walk(p, s->H, true)
+          ? mi::launch_f32_dq(s->D, q, k, v, dout, lse, delta, dq, p, stream)
+          : mi::launch_bwd_dq(s->dtype, s->D, q, k, v, dout, lse, delta, dq, p, stream);
   if (e != hipSuccess) return MI_ERR_LAUNCH;
   if (sp == SinkPass::kNone) return MI_OK;
   return status_of(mi::launch_sink_dq(s->dtype, s->D, q, k, v, dout, lse, delta, dq, p, stream));
@@ -411,8 +425,8 @@ int run_bwd(const void* q, const void* k, const void* v, const float* gate, cons
   if (o_res && !aligned16(o_res)) return MI_ERR_ALIGN;
   if (!q || !k || !v || !o || !dout || !lse || !delta || !dq || !dk || !dv) return MI_ERR_NULL;
   const mi::AttnParams p = params(s);
-  if (!gate && s->dtype != MI_F32) {
-    // 16-bit, no gate: the dQ kernel computes the delta pass itself and runs
+  if (!gate && (s->dtype != MI_F32 || mi::f32_split_walk(p, s->H, true))) {
+    // No gate, and a dQ kernel that can: the dQ kernel computes the delta pass itself and runs
     // first; dK/dV (and the sink pass) then read the planes it wrote.
     if (!aligned16(o) || !aligned16(delta)) return MI_ERR_ALIGN;
     if (!mi::sink_bwd_fusable(p)) {

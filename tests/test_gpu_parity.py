@@ -976,3 +976,43 @@ def test_random_shape_and_mask_sweep(case):
             assert err < tol, f"{tag}: {name} max|err| {err:.3e} >= {tol:.1e}"
         else:
             _parity.check(tag, name, a, b, dtype, extra=extra.get(name))
+
+
+# ---------------------------------------------------------------------------
+# float32: the split-walk kernels (attn_f32.hip) and the 128-row ones
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("T", [1, 31, 33, 127, 129, 161])
+@pytest.mark.parametrize("mode", ["causal", "noncausal", "window", "blocks"])
+def test_f32_split_walk_edges(D, T, mode):
+    """Row counts around the 32-row tiles and the four waves' shares (a wave with no
+    tile, one with two), a GQA group whose walk crosses heads, an LSE gradient."""
+    B, H, Hkv = 2, 6, 2
+    q, k, v, do = _rand(B, T, H, Hkv, D, torch.float32, seed=T * 3 + D)
+    dl = torch.randn(B, H, T, generator=torch.Generator().manual_seed(T))
+    causal, window, block = mode != "noncausal", 33 if mode == "window" else 0, \
+        7 if mode == "blocks" else 0
+    scale = 1.0 / math.sqrt(D)
+    xs = [t.cuda().requires_grad_() for t in (q, k, v)]
+    o, lse = fc.attn(*xs, causal, window, scale, block=block)
+    grads = torch.autograd.grad((o, lse), xs, (do.cuda(), dl.cuda()))
+    got = [t.detach().double().cpu().numpy() for t in (o, lse, *grads)]
+    ow, lw = orc.forward(q, k, v, scale, causal, window, block=block)
+    want = [ow, lw, *orc.backward(q, k, v, ow, lw, do, scale, causal, window, block=block,
+                                  dlse=dl)]
+    _compare(got, want, torch.float32, f"f32 split {mode} T{T} D{D}")
+
+
+@pytest.mark.parametrize("B,T,D,window", [(64, 100, 64, 0), (64, 127, 32, 0), (32, 300, 64, 40),
+                                          (24, 100, 128, 0)])
+def test_f32_full_chip_short_walks(B, T, D, window):
+    """Many heads with short walks: the 128-row float32 kernels (the launches that the
+    split walk leaves to them)."""
+    H = 12
+    q, k, v, do = _rand(B, T, H, H // 2, D, torch.float32, seed=T)
+    scale = 1.0 / math.sqrt(D)
+    got = _gpu(q, k, v, do, True, window, scale)
+    for b in (0, B // 2, B - 1):
+        sl = slice(b, b + 1)
+        want = _ref(q[sl], k[sl], v[sl], do[sl], True, window, scale)
+        _compare([g[sl] for g in got], want, torch.float32, f"f32 full chip B{B} T{T} D{D} b{b}")
