@@ -66,6 +66,7 @@ _DTYPE_CODE = {torch.float32: _capi.MI_F32, torch.float16: _capi.MI_F16,
                torch.bfloat16: _capi.MI_BF16}
 
 _lib = None
+_ext = None          # the C++ autograd nodes (csrc/autograd.cpp), imported with the library
 _load_error: str | None = None
 _load_attempted = False
 _mma_ok = False
@@ -110,7 +111,7 @@ def _load():
     Returns the ctypes library or None with ``_load_error`` set. Never raises:
     callers gate on ``is_available()``.
     """
-    global _lib, _load_error, _load_attempted, _mma_ok, _mma_error, _f32_ok, _f32_error
+    global _lib, _ext, _load_error, _load_attempted, _mma_ok, _mma_error, _f32_ok, _f32_error
     if _load_attempted:
         return _lib
     _load_attempted = True
@@ -129,11 +130,12 @@ def _load():
         return None
     try:
         lib = _capi.load()
-    except OSError as e:
-        _load_error = f"OSError: {e}"
+        from . import _mi_torch as ext
+    except (OSError, ImportError) as e:
+        _load_error = f"{type(e).__name__}: {e}"
         log.warning("libmi_attn.so did not load (%s)", _load_error)
         return None
-    _lib = lib
+    _lib, _ext = lib, ext
     _mma_ok, _mma_error = True, None
     for dt in MMA_DTYPES:
         ok, why = _probe_mfma(lib, dt)
@@ -341,7 +343,9 @@ class _AttnFn(torch.autograd.Function):
 
     The LSE tape [B,H,S] is saved for the backward, like the reference's
     ``_FlashAttnFn`` (``nanolab/flash_cuda.py:205-230``); its incoming
-    gradient folds into Delta inside the library.
+    gradient folds into Delta inside the library. ``_apply`` takes the same node
+    in C++ (``csrc/autograd.cpp``) wherever the call is plain eager; this
+    one is what a tracer can record.
     """
 
     @staticmethod
@@ -362,6 +366,19 @@ class _AttnFn(torch.autograd.Function):
         dq, dk, dv, dgate = _bwd(do, dlse, q, k, v, o, lse, ctx.causal, ctx.window, ctx.sinks,
                                  ctx.scale, gate, ctx.block, o_res)
         return dq, dk, dv, None, None, None, None, dgate, None
+
+
+def _recorded() -> bool:
+    """Whether a tracer records this call (``torch.jit.trace`` keeps a Python node as an
+    operator; Dynamo reads one): it then takes the Python autograd node."""
+    return torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
+
+
+def _apply(q, k, v, causal, window, sinks, scale, gate, block):
+    if _recorded():
+        return _AttnFn.apply(q, k, v, causal, window, sinks, scale, gate, block)
+    return _ext.attn(q, k, v, gate, causal, window, sinks, scale, block,
+                     _wants_residual(q, sinks, gate, window))
 
 
 def _prepare(q, k, v, causal, window, sinks, scale, use_mma, who, block=0):
@@ -436,12 +453,12 @@ def _run(q, k, v, causal, window, sinks, scale, dtype, use_mma, gate=None, block
         # fp32 arithmetic end to end on upcast copies; the casts are autograd ops.
         if not _f32_ok:
             raise RuntimeError(f"float32 path unavailable ({_f32_error})")
-        o, lse = _AttnFn.apply(q.float(), k.float(), v.float(), causal, window, sinks, scale,
-                               gate, block)
+        o, lse = _apply(q.float(), k.float(), v.float(), causal, window, sinks, scale, gate,
+                        block)
         return o.to(dtype), lse
     if dtype == torch.float32 and not _f32_ok:
         raise RuntimeError(f"float32 path unavailable ({_f32_error})")
-    return _AttnFn.apply(q, k, v, causal, window, sinks, scale, gate, block)
+    return _apply(q, k, v, causal, window, sinks, scale, gate, block)
 
 
 def _gate_of(gate, q, who):
