@@ -22,6 +22,8 @@
 // register layout itself is checked at load time by mi_mfma_probe.
 #pragma once
 
+#include <type_traits>
+
 #include "attn_common.h"
 
 namespace mi {
@@ -161,6 +163,30 @@ __device__ __forceinline__ typename Mfma32<T>::frag lds_frag_tr(const char* p0, 
   typedef short s16x8 __attribute__((ext_vector_type(8)));
   const s16x8 ab = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
   return __builtin_bit_cast(typename Mfma32<T>::frag, ab);
+}
+
+// The rounding residual of 8 accumulator values (registers base .. base+7)
+// against hi, their packed 16-bit fragment: (T)(x - (float)hi) per element.
+// bf16: hi back in float32 straight from the packed pairs (a bf16 is the upper
+// half of a float32; element 2i in the low half of word i), a shift or a mask
+// per element; f16: a conversion. hi + lo carries x to ~16 significant bits.
+template <typename T>
+__device__ __forceinline__ typename Mfma32<T>::frag lo_frag(const f32x16& acc, int base,
+                                                            typename Mfma32<T>::frag hi) {
+  typename Mfma32<T>::frag lo;
+  const u32x4 hw = __builtin_bit_cast(u32x4, hi);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float h;
+    if constexpr (std::is_same_v<T, __bf16>) {
+      const unsigned w = hw[e >> 1];
+      h = __builtin_bit_cast(float, (e & 1) ? (w & 0xffff0000u) : (w << 16));
+    } else {
+      h = (float)hi[e];
+    }
+    lo[e] = (T)(acc[base + e] - h);
+  }
+  return lo;
 }
 
 // Epilogue stores through LDS. Without it, a wave's 32 x D output rows leave

@@ -34,9 +34,9 @@
 //    LDS tile, prefetching the next block while it computes, so the loop
 //    needs no workgroup barrier;
 //  * fp32 inputs, and one-token steps with few query rows per kv head: VALU.
-//    A 32-column MFMA would be mostly padding there, and the step is a pure
-//    HBM stream. Lane groups over keys, 16 bytes per lane, several keys in
-//    flight per group.
+//    Lane groups over keys, 16 bytes per lane, several keys in flight per
+//    group. (Two to four 16-bit rows take the MFMA kernel where that measured
+//    faster: dec_small_mfma.)
 #include <type_traits>
 
 #include "attn16.h"
@@ -215,7 +215,11 @@ struct Dec16 {
 // one BN-key block held in LDS as natural K / V tiles (swizzled chunks, the
 // forward kernel's layout and fragment maps) plus, with a window, the keys'
 // positions.
-template <typename T, int D, bool SWA>
+// HL: P enters the PV product as two 16-bit terms, its rounding and the
+// rounding of the residual (~16 significant bits), for steps of a few rows,
+// whose probabilities the VALU kernel holds in fp32; the second MFMA is free
+// there (the step waits for K and V).
+template <typename T, int D, bool SWA, bool HL = false>
 struct Dec16Rows {
   using C = Dec16<D>;
   using M = Mfma32<T>;
@@ -318,11 +322,15 @@ struct Dec16Rows {
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
         const frag pb = pack_frag<T>(s[mt], ks * 8);
+        frag pl;
+        if constexpr (HL) pl = lo_frag<T>(s[mt], ks * 8, pb);
         const int roff = (32 * mt + 16 * ks) * D * 2;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-          oacc[dt] = M::mma(lds_frag_tr<T>(sV + vaddr[dt][0] + roff, sV + vaddr[dt][1] + roff),
-                            pb, oacc[dt]);
+        for (int dt = 0; dt < DT; ++dt) {
+          const frag vt = lds_frag_tr<T>(sV + vaddr[dt][0] + roff, sV + vaddr[dt][1] + roff);
+          oacc[dt] = M::mma(vt, pb, oacc[dt]);
+          if constexpr (HL) oacc[dt] = M::mma(vt, pl, oacc[dt]);
+        }
       }
   }
 };
@@ -374,7 +382,7 @@ struct Dec16Stage {
 // At most 32 query rows per kv head: each wave streams its own blocks (every
 // WS-th of the split) through its private LDS tile, with no workgroup barrier
 // in the loop, and the waves merge at the end.
-template <typename T, int D, bool SWA>
+template <typename T, int D, bool SWA, bool HL>
 __global__ void __launch_bounds__(64 * Dec16<D>::WS)
 attn_decode16_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const T* __restrict__ Vc,
                      const T* __restrict__ Kn, const T* __restrict__ Vn, T* __restrict__ O,
@@ -399,7 +407,7 @@ attn_decode16_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const T*
   char* sV = tiles[wave] + C::TILE;
   int* sP = reinterpret_cast<int*>(tiles[wave] + 2 * C::TILE);
 
-  Dec16Rows<T, D, SWA> st;
+  Dec16Rows<T, D, SWA, HL> st;
   st.init(p, Q, b, kvh, tile, lane);
   const DecRows rows = dec_rows<T>(p, Kc, Vc, Kn, Vn, b, kvh);
   Dec16Stage<T, D, 64> stage;
@@ -827,6 +835,24 @@ static void dec_geometry(DecParams& p) {
   p.nsplit = (nblk + p.bps - 1) / p.bps;
 }
 
+// Two to four 16-bit query rows per kv head, planned as the VALU kernel's units
+// (RT rows, BN-key blocks): whether the MFMA kernel runs them. The rows' dot
+// products and converted keys hold a lone VALU workgroup back, while an MFMA's
+// padded columns cost nothing; but its eight waves' tiles fill a CU's LDS (half
+// of it at D = 32), so it wins where the workgroups are one round of the chip,
+// and the VALU kernel's smaller ones beyond. One step, us, VALU -> MFMA (grid =
+// workgroups):
+//   grid 8    B1 H32/8 L1000 D128   30.3 -> 16.4    grid 320  B10 H32/8 L2048 D128  24.1 -> 27.9
+//   grid 128  B4 H24/8 L2048 D128   22.4 -> 15.4    grid 512  B8 H32/8 L4096 D128   30.5 -> 33.9
+//   grid 256  B4 H16/8 L4096 D128   23.9 -> 20.3    grid 512  B16 H16/8 L4096 D64   30.2 -> 32.5
+//   grid 192  B16 T2 H12 L1024 D64  19.8 -> 12.0    grid 640  B80 H32/8 L800 D64    28.5 -> 34.2
+//   grid 256  B8 H32/8 L4096 D64    24.2 -> 18.4    grid 512  B16 H16/8 L8192 D32   30.6 -> 28.6
+template <int D>
+static bool dec_small_mfma(const DecParams& p) {
+  const long long grid = (long long)p.B * p.Hkv * p.nsplit;
+  return p.R >= 2 && p.R <= kDecValuRows && grid <= (D <= 32 ? 512 : 256);
+}
+
 template <typename T, int D, int RT>
 static void launch_valu(dim3 grid, bool swa, const T* Q, const T* Kc, const T* Vc, const T* Kn,
                         const T* Vn, T* out, float* lse, float* ws, const DecParams& p,
@@ -857,8 +883,21 @@ static hipError_t launch_decode_t(const void* q, const void* kc, const void* vc,
       if constexpr (sizeof(T) == 4) launch_valu<T, D, 8>(grid, swa, Q, Kc, Vc, Kn, Vn, (T*)out, lse, ws, p, st);
       break;
     case kDecValuRows:
-      if constexpr (sizeof(T) == 2)
-        launch_valu<T, D, kDecValuRows>(grid, swa, Q, Kc, Vc, Kn, Vn, (T*)out, lse, ws, p, st);
+      if constexpr (sizeof(T) == 2) {
+        if (dec_small_mfma<D>(p)) {
+          DecParams m = p;   // the same key ranges in the MFMA kernel's blocks
+          static_assert(DecV<T, D, kDecValuRows>::BN % Dec16<D>::BN == 0, "whole blocks");
+          m.bps = p.bps * (DecV<T, D, kDecValuRows>::BN / Dec16<D>::BN);
+          if (swa)
+            hipLaunchKernelGGL((attn_decode16_kernel<T, D, true, true>), grid, dim3(64 * Dec16<D>::WS),
+                               0, st, Q, Kc, Vc, Kn, Vn, (T*)out, lse, ws, m);
+          else
+            hipLaunchKernelGGL((attn_decode16_kernel<T, D, false, true>), grid, dim3(64 * Dec16<D>::WS),
+                               0, st, Q, Kc, Vc, Kn, Vn, (T*)out, lse, ws, m);
+        } else {
+          launch_valu<T, D, kDecValuRows>(grid, swa, Q, Kc, Vc, Kn, Vn, (T*)out, lse, ws, p, st);
+        }
+      }
       break;
     default:
       if constexpr (sizeof(T) == 2) {
@@ -870,10 +909,10 @@ static hipError_t launch_decode_t(const void* q, const void* kc, const void* vc,
           hipLaunchKernelGGL((attn_decode16_wg_kernel<T, D, false>), grid, dim3(256), 0, st, Q, Kc,
                              Vc, Kn, Vn, (T*)out, lse, ws, p);
         else if (swa)
-          hipLaunchKernelGGL((attn_decode16_kernel<T, D, true>), grid, dim3(64 * Dec16<D>::WS), 0, st, Q, Kc, Vc,
+          hipLaunchKernelGGL((attn_decode16_kernel<T, D, true, false>), grid, dim3(64 * Dec16<D>::WS), 0, st, Q, Kc, Vc,
                              Kn, Vn, (T*)out, lse, ws, p);
         else
-          hipLaunchKernelGGL((attn_decode16_kernel<T, D, false>), grid, dim3(64 * Dec16<D>::WS), 0, st, Q, Kc,
+          hipLaunchKernelGGL((attn_decode16_kernel<T, D, false, false>), grid, dim3(64 * Dec16<D>::WS), 0, st, Q, Kc,
                              Vc, Kn, Vn, (T*)out, lse, ws, p);
       }
   }

@@ -544,3 +544,29 @@ def test_window_commit_equals_boolean_indexing(dtype, Lc, T, window, sinks, evic
         attn_cached(q, k, v, cache, True, True, window=window, sinks=sinks)
     assert torch.equal(cache["pos"], kpos[live]) and cache["end"] == start + T
     assert torch.equal(cache["k"], kf[:, :, live]) and torch.equal(cache["v"], vf[:, :, live])
+
+
+# (B, T, cached, H, Hkv): two to four query rows per kv head, on both sides of the grid
+# where the MFMA kernel takes them (one round of workgroups), split and unsplit, key
+# counts around its 32 / 64-key blocks.
+SMALL_ROWS = [(1, 1, 31, 4, 2), (1, 2, 64, 3, 3), (2, 1, 700, 6, 2), (1, 4, 65, 2, 2),
+              (1, 1, 9000, 8, 2), (3, 2, 2100, 4, 2), (70, 1, 40, 32, 8)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES[1:], ids=lambda d: str(d).replace("torch.", ""))
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("shape", SMALL_ROWS, ids=lambda s: "B%dT%dL%dH%d_%d" % s)
+@pytest.mark.parametrize("mode", ["causal", "bidir", "window"])
+def test_decode_two_to_four_rows(dtype, D, shape, mode):
+    B, T, Lc, H, Hkv = shape
+    g = np.random.default_rng(Lc * 3 + D)
+    q = g.standard_normal((B, T, H, D)) * 2
+    k, v = (g.standard_normal((B, T, Hkv, D)) for _ in range(2))
+    cache = {n: g.standard_normal((B, Hkv, Lc, D)) for n in "kv"}
+    window, sinks = (0, 0) if mode != "window" else (min(Lc, 40) + T, 3)
+    if mode == "window":
+        cache["end"] = Lc
+    gate = g.standard_normal((B, T, H)) if T == 2 else None
+    _step(q, k, v, cache, dtype, mode != "bidir", window=window, sinks=sinks, gate=gate,
+          tag=f"decode rows {dtype} D{D} {shape} {mode}")
