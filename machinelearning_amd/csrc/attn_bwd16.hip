@@ -97,6 +97,14 @@ __host__ __device__ inline long long split_pitch(int S) { return (S + 127LL) / 1
 // backward then runs dQ before dK/dV and needs no separate delta pass. Each
 // query row is owned by exactly one lane pair, so every plane entry is written
 // once.
+//
+// With p.gate (FD, no LSE gradient) O and dO are those of the gated output y =
+// sigma O: dS = P (sigma dO V^T - Delta) = (sigma P)(dO V^T - Delta / sigma), so
+// both kernels run on dO itself with the planes Delta / sigma and (ln sigma -
+// LSE) / scale; the gate's gradient (1 - sigma) rowsum(dO * y) is a row scalar.
+// That drops the delta launch and the scaled copy of dO. Logits are taken as at
+// least -85 (sigma 1e-37): below, sigma P is gone from any 16-bit result while
+// Delta / sigma stays finite.
 // ---------------------------------------------------------------------------
 template <typename T, int D, bool BLK, bool FD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2, 8)))
@@ -138,10 +146,12 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
   // This row's LSE (and LSE gradient), loaded up front: with O by DMA the
   // delta is finished only after the ring's first wait.
   const long long ridx = ((long long)b * p.H + h) * p.S + qi;
-  float Lrow = 0.f, dlrow = 0.f;
+  float Lrow = 0.f, dlrow = 0.f, zrow = 0.f;
+  const long long zidx = ((long long)b * p.S + qi) * p.H + h;
   if (FD && qi < p.S) {
     Lrow = LSE[ridx];
     if (p.dlse) dlrow = p.dlse[ridx];
+    if (p.gate) zrow = p.gate[zidx];
   }
   // Fused delta, given this lane's partial dot product of dO and O (head dims
   // {16 ds + 8 g + e} of row qi; the lane 32 away holds the other half).
@@ -149,7 +159,13 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
     Dq = halves_sum(part);
     if (qi < p.S) {
       const long long idx = ridx;
-      const float L = Lrow;
+      float L = Lrow;
+      if (p.gate) {
+        const float e = 1.f + __expf(zrow < -85.f ? 85.f : -zrow);   // 1 / sigma; NaN stays
+        if (g == 0) p.dgate[zidx] = (1.f - 1.f / (1.f + __expf(-zrow))) * Dq;
+        Dq *= e;
+        L += logf(e);
+      }
       L2 = L * kLog2e;
       Dq -= dlrow;
       if (g == 0) {

@@ -164,6 +164,7 @@ mi::AttnParams params(const mi_attn_shape* s) {
   p.q_rs = (long long)s->H * s->D;
   p.kv_rs = (long long)s->Hkv * s->D;
   p.gate = nullptr;
+  p.dgate = nullptr;
   p.o = nullptr;
   p.dlse = nullptr;
   p.ws_out = nullptr;
@@ -363,7 +364,7 @@ int run_dkdv(const void* q, const void* k, const void* v, const void* dout, cons
 int run_dq(const void* q, const void* k, const void* v, const void* dout, const float* lse,
            const float* delta, void* dq, const mi_attn_shape* s, hipStream_t stream,
            SinkPass sp, const void* o = nullptr, const float* dlse = nullptr,
-           const void* o_res = nullptr) {
+           const void* o_res = nullptr, const float* gate = nullptr, float* dgate = nullptr) {
   if (!q || !k || !v || !dout || !lse || !delta || !dq) return MI_ERR_NULL;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(dout) || !aligned16(dq) ||
       (o && !aligned16(o)))
@@ -374,6 +375,8 @@ int run_dq(const void* q, const void* k, const void* v, const void* dout, const 
     p.dlse = dlse;
     p.ws_out = const_cast<float*>(delta);
     p.o_res = const_cast<void*>(o_res);
+    p.gate = gate;
+    p.dgate = dgate;
   }
   const hipError_t e =
       s->dtype != MI_F32
@@ -539,6 +542,23 @@ int mi_attn_bwd_gated(const void* q, const void* k, const void* v, const float* 
   if (!gate || !dout_attn || !dgate) return MI_ERR_NULL;
   return run_bwd(q, k, v, gate, o, dout, lse, dlse, delta, dout_attn, dq, dk, dv, dgate, s,
                  stream);
+}
+
+int mi_attn_bwd_gated_direct(const void* q, const void* k, const void* v, const float* gate,
+                             const void* o, const void* dout, const float* lse, float* delta,
+                             void* dq, void* dk, void* dv, float* dgate, const mi_attn_shape* s,
+                             hipStream_t stream) {
+  const int st = validate(s);
+  if (st) return st;
+  if (s->dtype == MI_F32) return MI_ERR_DTYPE;
+  if (empty(s)) return MI_OK;
+  if (!q || !k || !v || !gate || !o || !dout || !lse || !delta || !dq || !dk || !dv || !dgate)
+    return MI_ERR_NULL;
+  if (!aligned16(o) || !aligned16(delta)) return MI_ERR_ALIGN;
+  const int r = run_dq(q, k, v, dout, lse, delta, dq, s, stream, SinkPass::kNone, o, nullptr, nullptr,
+                       gate, dgate);
+  if (r) return r;
+  return run_dkdv(q, k, v, dout, lse, delta, dk, dv, s, stream, SinkPass::kNone);
 }
 
 namespace {

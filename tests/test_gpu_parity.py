@@ -1016,3 +1016,41 @@ def test_f32_full_chip_short_walks(B, T, D, window):
         sl = slice(b, b + 1)
         want = _ref(q[sl], k[sl], v[sl], do[sl], True, window, scale)
         _compare([g[sl] for g in got], want, torch.float32, f"f32 full chip B{B} T{T} D{D} b{b}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,mode", [(32, "blocks"), (64, "window+sinks"), (64, "noncausal"),
+                                    (128, "causal")])
+def test_gated_backward_without_dout_copy(dtype, D, mode):
+    """The gated backward that folds sigma into the planes: logits over the whole range
+    (sigma 1 down to underflow), at the plain bounds and finite; and an LSE gradient, which
+    takes the other route, adds to it."""
+    B, T, H, Hkv = 2, 150, 4, 2
+    q, k, v, do = _rand(B, T, H, Hkv, D, dtype, seed=D)
+    g = torch.Generator().manual_seed(D)
+    z = torch.randn(B, T, H, generator=g)
+    z[:, ::5] *= 30
+    z[:, 3::17] = -200.0
+    z[:, 4::17] = 200.0
+    causal, window, sinks, block = mode != "noncausal", *((24, 3) if "sinks" in mode else (0, 0)), \
+        20 if mode == "blocks" else 0
+    scale = 1.0 / math.sqrt(D)
+    xs = [t.cuda().requires_grad_() for t in (q, k, v, z)]
+    y, lse = fc.attn(*xs[:3], causal, window, scale, sinks=sinks, gate=xs[3], block=block)
+    grads = torch.autograd.grad(y, xs, do.cuda(), retain_graph=True)
+    o, lw = orc.forward(q, k, v, scale, causal, window, sinks=sinks, block=block)
+    sg = 1 / (1 + np.exp(-z.double().numpy()))
+    dof = do.double().numpy() * sg[..., None]
+    want = [o * sg[..., None], lw, *orc.backward(q, k, v, o, lw, dof, scale, causal, window,
+                                                 sinks=sinks, block=block)]
+    got = [t.detach().double().cpu().numpy() for t in (y, lse, *grads[:3])]
+    _compare(got, want, dtype, f"gated direct {mode} D{D} {dtype}")
+    dz = (do.double().numpy() * o).sum(-1) * sg * (1 - sg)
+    _parity.check(f"gated direct {mode} D{D} {dtype}", "dgate", grads[3].double().cpu().numpy(), dz,
+                  dtype)
+    dl = torch.randn(B, H, T, generator=g)
+    both = torch.autograd.grad((y, lse), xs[:3], (do.cuda(), dl.cuda()))
+    want = [None, None, *orc.backward(q, k, v, o, lw, dof, scale, causal, window, sinks=sinks,
+                                      block=block, dlse=dl)]
+    for n, a, b in zip(("dQ", "dK", "dV"), both, want[2:]):
+        _parity.check(f"gated + dLSE {mode} D{D} {dtype}", n, a.double().cpu().numpy(), b, dtype)
