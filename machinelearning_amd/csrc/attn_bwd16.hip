@@ -104,7 +104,8 @@ __host__ __device__ inline long long split_pitch(int S) { return (S + 127LL) / 1
 // LSE) / scale; the gate's gradient (1 - sigma) rowsum(dO * y) is a row scalar.
 // That drops the delta launch and the scaled copy of dO. Logits are taken as at
 // least -85 (sigma 1e-37): below, sigma P is gone from any 16-bit result while
-// Delta / sigma stays finite.
+// Delta / sigma stays finite. (Board shape, gated step: 166.0 -> 155.9 us, the
+// ungated one 154.4; f16 rounding of sigma dO gone.)
 // ---------------------------------------------------------------------------
 template <typename T, int D, bool BLK, bool FD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2, 8)))
