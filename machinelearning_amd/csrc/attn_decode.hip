@@ -261,13 +261,15 @@ struct Dec16Rows {
     key_hi = p.causal ? min(p.Lk - 1, p.Lc + t) : p.Lk - 1;
   }
 
-  // Keys [k0, k0 + BN) from LDS.
+  // Keys [k0, k0 + NB BN) from LDS, NB blocks adjacent there. Two blocks' scores and
+  // maxima do not wait for each other; the blocks then enter the running sums one
+  // by one, with the maximum at their own block, as one call each would.
+  template <int NB = 1>
   __device__ __forceinline__ void block(const DecParams& p, const char* sK, const char* sV,
                                         const int* sP, int k0) {
-    const float c = p.scale_log2;
-    f32x16 s[MT];
+    f32x16 s[NB * MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
+    for (int mt = 0; mt < NB * MT; ++mt) {
       s[mt] = zero16();
 #pragma unroll
       for (int ds = 0; ds < DS; ++ds)
@@ -276,7 +278,7 @@ struct Dec16Rows {
     // Masks. Register r of half mt is key k0 + 32 mt + crow(r, g).
     if constexpr (SWA) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+      for (int mt = 0; mt < NB * MT; ++mt)
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
           const int kb = 32 * mt + 8 * jj + 4 * g;
@@ -286,28 +288,45 @@ struct Dec16Rows {
           for (int i = 0; i < 4; ++i)
             if (!dec_visible<true>(p, k0 + kb + i, kps[i], t)) s[mt][4 * jj + i] = -INFINITY;
         }
-    } else if (k0 + BN - 1 > key_hi) {
+    } else if (k0 + NB * BN - 1 > key_hi) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) mask_above(s[mt], key_hi - (k0 + mt * 32 + 4 * g), -INFINITY);
+      for (int mt = 0; mt < NB * MT; ++mt)
+        mask_above(s[mt], key_hi - (k0 + mt * 32 + 4 * g), -INFINITY);
     }
     // Online softmax: the lane owns query row l32 (its keys in both halves
     // of the wave), so the statistics are lane scalars.
-    float mx = s[0][0];
+    float mx[NB];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int b = 0; b < NB; ++b) {
+      mx[b] = s[b * MT][0];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mx = __builtin_elementwise_maximum(mx, s[mt][i]);
-    if (wave_any(mx > m_run)) {
-      const float m_new = fmaxf(m_run, halves_max(mx));
-      const float alpha = fast_exp2((m_run - m_new) * c);
-      l_run *= alpha;
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
-      m_run = m_new;
+        for (int i = 0; i < 16; ++i) mx[b] = __builtin_elementwise_maximum(mx[b], s[b * MT + mt][i]);
     }
-    const float mc = m_run * c;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if (wave_any(mx[b] > m_run)) raise(p, mx[b]);
+      probs(p, s + b * MT);
+      pv(s + b * MT, sV + b * C::TILE);
+    }
+  }
+
+  // A new running maximum: the sums so far, rescaled.
+  __device__ __forceinline__ void raise(const DecParams& p, float mx) {
+    const float m_new = fmaxf(m_run, halves_max(mx));
+    const float alpha = fast_exp2((m_run - m_new) * p.scale_log2);
+    l_run *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
+    m_run = m_new;
+  }
+
+  // A block's scores -> probabilities, and their sum.
+  __device__ __forceinline__ void probs(const DecParams& p, f32x16* s) {
+    const float c = p.scale_log2, mc = m_run * c;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -316,7 +335,10 @@ struct Dec16Rows {
         s[mt][i] = pv;
         l_run += pv;
       }
-    // O^T += V^T P^T over 16-key chunks.
+  }
+
+  // O^T += V^T P^T of a block, over 16-key chunks.
+  __device__ __forceinline__ void pv(const f32x16* s, const char* sV) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -453,9 +475,19 @@ attn_decode16_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const T*
 // More than 32 query rows per kv head (block verifies and drafts with GQA):
 // the workgroup's four waves own four consecutive 32-row tiles of one
 // (batch, kv head) and share every key block, staged once per workgroup
-// into a double-buffered LDS tile with one barrier per block. (Per-wave
-// streaming would read the keys once per 32-row tile.) Each wave then
-// writes its own rows: the output, or its split partial.
+// into LDS. (Per-wave streaming would read the keys once per 32-row tile.)
+// Bound by each wave's serial chain per step (LDS reads, MFMAs, max, exp,
+// MFMAs), with one or two waves per SIMD to hide it: without a window a step
+// takes two blocks, brought by LDS-DMA during the step before. Against one
+// block per step, double-buffered through registers (as still with a window,
+// whose visibility depends on each key's position), results the same bit for
+// bit: [8, 16, 32 / 8, 64] on 4096 keys 24.9 -> 23.2 us, [4, 64, 8 / 8, 64] on
+// 2000 24.0 -> 22.3, [4, 16, 12 / 4, 128] on 1500 28.5 -> 26.3, [2, 300, 8 / 4,
+// 128] on none 15.1 -> 14.3; [8, 32, 32 / 8, 128] on 4096, two workgroups on
+// every CU, stays at 41. LDS-DMA alone, one block per step: 23.9, 23.5, 27.4
+// and 16.5. One maximum for both blocks would give 22.3, 21.6 and 24.6, but P
+// is then exactly 1 less often, and the error grows by 0.5%.
+// Each wave then writes its own rows: the output, or its split partial.
 template <typename T, int D, bool SWA>
 __global__ void __launch_bounds__(256)
 attn_decode16_wg_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const T* __restrict__ Vc,
@@ -463,7 +495,10 @@ attn_decode16_wg_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const
                         float* __restrict__ LSE, float* __restrict__ ws, DecParams p) {
   using C = Dec16<D>;
   constexpr int W = C::W, BN = C::BN, DT = C::DT;
-  __shared__ __attribute__((aligned(1024))) char tiles[2][2 * C::TILE + 256];
+  // With a window a double buffer of K tile, V tile and the keys' positions;
+  // else a ring of four K tiles, then of four V tiles.
+  constexpr int NS = SWA ? 2 : 4;
+  __shared__ __attribute__((aligned(1024))) char tiles[NS][2 * C::TILE + (SWA ? 256 : 0)];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ngrp = (p.ntiles + W - 1) / W;
@@ -480,15 +515,70 @@ attn_decode16_wg_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const
 
   const int nblk = (p.Lk + BN - 1) / BN;
   const int blk0 = split * p.bps, blk1 = min(nblk, blk0 + p.bps);
-  if (blk0 < blk1) stage.load(p, rows, blk0, tid, SWA);
-  for (int blk = blk0; blk < blk1; ++blk) {
-    // Buffer (blk & 1) was last read in block blk - 2; every wave passed the
-    // barrier of block blk - 1 after that, so it is free.
-    char* buf = tiles[(blk - blk0) & 1];
-    stage.store(buf, buf + C::TILE, reinterpret_cast<int*>(buf + 2 * C::TILE), tid, SWA);
-    __syncthreads();
-    if (blk + 1 < blk1) stage.load(p, rows, blk + 1, tid, SWA);
-    st.block(p, buf, buf + C::TILE, reinterpret_cast<const int*>(buf + 2 * C::TILE), blk * BN);
+  if constexpr (SWA) {
+    if (blk0 < blk1) stage.load(p, rows, blk0, tid, SWA);
+    for (int blk = blk0; blk < blk1; ++blk) {
+      // Buffer (blk & 1) was last read in block blk - 2; every wave passed the
+      // barrier of block blk - 1 after that, so it is free.
+      char* buf = tiles[(blk - blk0) & 1];
+      stage.store(buf, buf + C::TILE, reinterpret_cast<int*>(buf + 2 * C::TILE), tid, SWA);
+      __syncthreads();
+      if (blk + 1 < blk1) stage.load(p, rows, blk + 1, tid, SWA);
+      st.block(p, buf, buf + C::TILE, reinterpret_cast<const int*>(buf + 2 * C::TILE), blk * BN);
+    }
+  } else {
+    // Two blocks per barrier and softmax step, the next two on their way into LDS
+    // while these are computed. Blocks of cached keys come by LDS-DMA, the few
+    // that reach into the active block through registers; of an empty cache, all
+    // by LDS-DMA (rows Hkv D apart; keys past Lk lie past the resource and are
+    // zeroed). One kind per launch: chosen per block it costs a third of the gain.
+    constexpr int LPW = C::TILE / 4096;      // DMA instructions per wave per tensor
+    const bool fresh = p.Lc == 0;
+    const int ld = fresh ? p.Hkv * D : D, dma_end = fresh ? nblk : p.Lc / BN;
+    const char* kb = static_cast<const char*>(fresh ? rows.kn : rows.kc);
+    const char* vb = static_cast<const char*>(fresh ? rows.vn : rows.vc);
+    unsigned off[LPW];
+#pragma unroll
+    for (int j = 0; j < LPW; ++j) {
+      const int slot = (4 * j + wave) * 64 + lane, row = slot / C::CH;
+      off[j] = (unsigned)(row * ld + ((slot % C::CH) ^ swz<D>(row)) * 8) * 2u;
+    }
+    auto issue = [&](int blk) __attribute__((always_inline)) {
+      char* kbuf = tiles[0] + ((blk - blk0) & 3) * C::TILE;
+      char* vbuf = kbuf + 4 * C::TILE;
+      if (blk < dma_end) {
+        const int k0 = blk * BN;
+        const long long at = (long long)k0 * ld * 2;
+        const unsigned len = (unsigned)((min(BN, p.Lk - k0) - 1) * ld + D) * 2u;
+        const Rsrc rk = make_rsrc(kb + at, len);
+        const Rsrc rv = make_rsrc(vb + at, len);
+        const unsigned m0 = lds_u32(kbuf + wave * 1024);
+#pragma unroll
+        for (int j = 0; j < LPW; ++j) {
+          dma16_buf(rk, off[j], m0 + (unsigned)(4096 * j));
+          dma16_buf(rv, off[j], m0 + (unsigned)(4 * C::TILE + 4096 * j));
+        }
+      } else {
+        int id = tid;
+        asm volatile("" : "+v"(id));   // its addresses are made here, not held
+        stage.load(p, rows, blk, id, false);
+        stage.store(kbuf, vbuf, nullptr, id, false);
+      }
+    };
+    if (blk0 < blk1) issue(blk0);
+    if (blk0 + 1 < blk1) issue(blk0 + 1);
+    // Retires the Q loads where the compiler sees it (else it would drain the
+    // ring before each block's first MFMA).
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    for (int blk = blk0; blk < blk1; blk += 2) {
+      wait_vm<0>();
+      lds_barrier();   // and every wave has finished the slots refilled now
+      if (blk + 2 < blk1) issue(blk + 2);
+      if (blk + 3 < blk1) issue(blk + 3);
+      const char* kbuf = tiles[0] + ((blk - blk0) & 3) * C::TILE;
+      if (blk + 1 < blk1) st.template block<2>(p, kbuf, kbuf + 4 * C::TILE, nullptr, blk * BN);
+      else st.block(p, kbuf, kbuf + 4 * C::TILE, nullptr, blk * BN);
+    }
   }
 
   // Each wave's rows: lane (l32, g) holds head dims dt*32 + 8jj + 4g + 0..3.

@@ -570,3 +570,24 @@ def test_decode_two_to_four_rows(dtype, D, shape, mode):
     gate = g.standard_normal((B, T, H)) if T == 2 else None
     _step(q, k, v, cache, dtype, mode != "bidir", window=window, sinks=sinks, gate=gate,
           tag=f"decode rows {dtype} D{D} {shape} {mode}")
+
+
+# (B, T, cached, H, Hkv): more than 32 query rows per kv head, which share blocks staged
+# two at a time: an empty cache, a last pair of one block, one block with keys of both
+# the cache and the step, a cache that ends on a block, splits.
+MANY_ROWS = [(1, 33, 0, 2, 2), (2, 70, 0, 4, 2), (1, 40, 1, 3, 3), (2, 17, 64, 8, 4),
+             (1, 34, 127, 2, 1), (1, 64, 130, 4, 2), (1, 9, 5001, 8, 2), (3, 33, 160, 2, 2)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES[1:], ids=lambda d: str(d).replace("torch.", ""))
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("shape", MANY_ROWS, ids=lambda s: "B%dT%dL%dH%d_%d" % s)
+@pytest.mark.parametrize("causal", [True, False], ids=["causal", "bidir"])
+def test_decode_more_than_32_rows(dtype, D, shape, causal):
+    B, T, Lc, H, Hkv = shape
+    g = np.random.default_rng(Lc * 3 + D)
+    q = g.standard_normal((B, T, H, D)) * 2
+    k, v = (g.standard_normal((B, T, Hkv, D)) for _ in range(2))
+    cache = {n: g.standard_normal((B, Hkv, Lc, D)) for n in "kv"}
+    _step(q, k, v, cache, dtype, causal, tag=f"decode many rows {dtype} D{D} {shape} {causal}")
