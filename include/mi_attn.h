@@ -62,7 +62,7 @@
 extern "C" {
 #endif
 
-#define MI_ATTN_ABI_VERSION 11
+#define MI_ATTN_ABI_VERSION 12
 
 #if defined(__GNUC__)
 #define MI_API __attribute__((visibility("default")))
@@ -202,23 +202,14 @@ MI_API int mi_attn_fwd_gated(const void* q, const void* k, const void* v, const 
  * of that output. `dout_attn` is a caller-owned [B,S,H,D] buffer of `dtype`
  * (16-byte aligned) that receives sigmoid(gate) * dout, the attention output's
  * gradient, which the dK/dV and dQ passes read; `dgate` [B,S,H] float32
- * receives the gate logits' gradient (1 - sigmoid) * rowsum(dout * o). */
+ * receives the gate logits' gradient (1 - sigmoid) * rowsum(dout * o).
+ * float16 / bfloat16: the dQ kernel writes both, with the bits of
+ * mi_attn_bwd_delta_gated; float32 launches that pass. */
 MI_API int mi_attn_bwd_gated(const void* q, const void* k, const void* v, const float* gate,
                              const void* o, const void* dout, const float* lse,
                              const float* dlse, float* delta, void* dout_attn, void* dq,
                              void* dk, void* dv, float* dgate, const mi_attn_shape* s,
                              hipStream_t stream);
-
-/* The gated backward without an LSE gradient, float16 / bfloat16 (others:
- * MI_ERR_DTYPE), in two launches and without dout_attn: with sigma = sigmoid(gate),
- * dS = sigma P (dout V^T - Delta / sigma) and dV = (sigma P)^T dout, so the planes
- * carry Delta / sigma and (ln sigma - LSE) / scale and the kernels read dout
- * itself. Logits below -85 count as -85 there (sigma 1e-37). Gradients differ
- * from mi_attn_bwd_gated's by the rounding of dout_attn. */
-MI_API int mi_attn_bwd_gated_direct(const void* q, const void* k, const void* v, const float* gate,
-                                    const void* o, const void* dout, const float* lse,
-                                    float* delta, void* dq, void* dk, void* dv, float* dgate,
-                                    const mi_attn_shape* s, hipStream_t stream);
 
 /* Stage 1 of the gated backward: mi_attn_bwd_delta plus dout_attn and dgate
  * (as above). Stages 2 and 3 are then mi_attn_bwd_dkdv / mi_attn_bwd_dq with

@@ -12,7 +12,7 @@ import ctypes
 import pathlib
 
 LIB_PATH = pathlib.Path(__file__).resolve().parent / "libmi_attn.so"
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 MI_F32, MI_F16, MI_BF16 = 0, 1, 2
 
@@ -91,7 +91,6 @@ SIGNATURES = {
     "mi_attn_bwd_res": (ctypes.c_int, [_P] * 12 + [_SHAPE, _P]),
     "mi_attn_fwd_gated": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _SHAPE, _P]),
     "mi_attn_bwd_gated": (ctypes.c_int, [_P] * 14 + [_SHAPE, _P]),
-    "mi_attn_bwd_gated_direct": (ctypes.c_int, [_P] * 12 + [_SHAPE, _P]),
     "mi_attn_bwd_delta_gated": (ctypes.c_int, [_P] * 8 + [_SHAPE, _P]),
     "mi_attn_bwd_dkdv": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _SHAPE, _P]),
     "mi_attn_bwd_dq": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _SHAPE, _P]),

@@ -98,16 +98,18 @@ __host__ __device__ inline long long split_pitch(int S) { return (S + 127LL) / 1
 // query row is owned by exactly one lane pair, so every plane entry is written
 // once.
 //
-// With p.gate (FD, no LSE gradient) O and dO are those of the gated output y =
-// sigma O: dS = P (sigma dO V^T - Delta) = (sigma P)(dO V^T - Delta / sigma), so
-// both kernels run on dO itself with the planes Delta / sigma and (ln sigma -
-// LSE) / scale; the gate's gradient (1 - sigma) rowsum(dO * y) is a row scalar.
-// That drops the delta launch and the scaled copy of dO. Logits are taken as at
-// least -85 (sigma 1e-37): below, sigma P is gone from any 16-bit result while
-// Delta / sigma stays finite. (Board shape, gated step: 166.0 -> 155.9 us, the
-// ungated one 154.4; f16 rounding of sigma dO gone.)
+// GATE (with FD): O and dO are those of the gated output y = sigma O. The kernel
+// then also does the rest of the delta pass (attn_bwd_delta_kernel): dS = P
+// (sigma dO V^T - Delta) takes the rows sigma * dO, rounded to T, which it
+// writes to p.doe for dK/dV, and the gate's gradient is (1 - sigma) rowsum(dO * y).
+// Sums and roundings are those of the delta pass, so the results are its bits.
+// (sigma stays with dO: sigma P would leave float16's range at logits of -4 and
+// bfloat16's near -80, where sigma * dO is still in it.) Backward with the delta
+// launch -> without, us: board shape bf16 135.5 -> 127.0 (ungated 121.4), f16
+// 136.5 -> 130.0; f16 B5 S777 H9/3 D64, blocks of 32: 51.0 -> 47.3; bf16 B2
+// S4096 H16 D128: 547 -> 537.
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool BLK, bool FD>
+template <typename T, int D, bool BLK, bool FD, bool GATE = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2, 8)))
 attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
                      const T* __restrict__ dO, const float* __restrict__ LSE,
@@ -147,12 +149,11 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
   // This row's LSE (and LSE gradient), loaded up front: with O by DMA the
   // delta is finished only after the ring's first wait.
   const long long ridx = ((long long)b * p.H + h) * p.S + qi;
-  float Lrow = 0.f, dlrow = 0.f, zrow = 0.f;
-  const long long zidx = ((long long)b * p.S + qi) * p.H + h;
+  float Lrow = 0.f, dlrow = 0.f, sg = 1.f;
   if (FD && qi < p.S) {
     Lrow = LSE[ridx];
     if (p.dlse) dlrow = p.dlse[ridx];
-    if (p.gate) zrow = p.gate[zidx];
+    if constexpr (GATE) sg = gate_sigmoid(p, b, qi, h);
   }
   // Fused delta, given this lane's partial dot product of dO and O (head dims
   // {16 ds + 8 g + e} of row qi; the lane 32 away holds the other half).
@@ -160,12 +161,16 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
     Dq = halves_sum(part);
     if (qi < p.S) {
       const long long idx = ridx;
-      float L = Lrow;
-      if (p.gate) {
-        const float e = 1.f + __expf(zrow < -85.f ? 85.f : -zrow);   // 1 / sigma; NaN stays
-        if (g == 0) p.dgate[zidx] = (1.f - 1.f / (1.f + __expf(-zrow))) * Dq;
-        Dq *= e;
-        L += logf(e);
+      const float L = Lrow;
+      if constexpr (GATE) {
+        if (g == 0) p.dgate[((long long)b * p.S + qi) * p.H + h] = (1.f - sg) * Dq;
+        T* doe = reinterpret_cast<T*>(p.doe) + ((long long)b * p.S + qi) * p.q_rs + (long long)h * D;
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) dof[ds][e] = (T)((float)dof[ds][e] * sg);
+          *reinterpret_cast<frag*>(doe + ds * 16 + g * 8) = dof[ds];
+        }
       }
       L2 = L * kLog2e;
       Dq -= dlrow;
@@ -173,6 +178,27 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
         p.ws_out[idx] = Dq;
         p.ws_out[(long long)p.B * p.H * p.S + idx] = L * (-1.f / p.scale);
       }
+    }
+  };
+  // This lane's partial of rowsum(dO * O), chunk ds of O at a time. GATE: each
+  // chunk summed by itself, the chunks in the delta pass's order.
+  float part = 0.f, chunk[GATE ? DS : 1];
+  auto add_chunk = [&](int ds, const frag& of) __attribute__((always_inline)) {
+    float x = GATE ? 0.f : part;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x = fmaf((float)of[e], (float)dof[ds][e], x);
+    if constexpr (GATE) chunk[ds] = x;
+    else part = x;
+  };
+  auto row_part = [&]() __attribute__((always_inline)) {
+    if constexpr (GATE) {
+#pragma unroll
+      for (int x = DS / 2; x >= 1; x >>= 1)
+#pragma unroll
+        for (int ds = 0; ds < x; ++ds) chunk[ds] += chunk[ds + x];
+      return chunk[0];
+    } else {
+      return part;
     }
   };
   // O of the workgroup's 128 rows by LDS-DMA into ring slot NS - 1, which the
@@ -186,7 +212,6 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
   if constexpr (FD) {
     const long long hoff = (long long)b * p.S * p.q_rs + (long long)h * D;
     const T* Ob = reinterpret_cast<const T*>(p.o) + hoff;
-    float part = 0.f;
     if (o_dma) {
       const RowTiles tOr = row_tiles(p.o, b, p.S, p.q_rs, h, D);
       unsigned ooff[C::LPW];
@@ -199,7 +224,7 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
         for (int j = 0; j < C::LPW; ++j)
           dma16_buf(ro, ooff[j], m0o + (unsigned)(half * C::TILE + 4096 * j));
       }
-    } else if (p.o_res) {
+    } else if (!GATE && p.o_res) {
       // O as stored plus its rounding residual: Delta from O to ~16 bits
       // (with O alone, its 8-bit rounding enters every dS of the row).
       const T* Rb = reinterpret_cast<const T*>(p.o_res) + hoff;
@@ -216,11 +241,10 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
       for (int ds = 0; ds < DS; ++ds) {
         const frag of = (qi < p.S) ? ld_frag<T>(Ob + (long long)qi * p.q_rs + ds * 16 + g * 8)
                                    : zero_frag<T>();
-#pragma unroll
-        for (int e = 0; e < 8; ++e) part = fmaf((float)of[e], (float)dof[ds][e], part);
+        add_chunk(ds, of);
       }
     }
-    if (!o_dma) finish_delta(part);
+    if (!o_dma) finish_delta(row_part());
   } else if (qi < p.S) {
     const long long idx = ((long long)b * p.H + h) * p.S + qi;
     L2 = LSE[idx] * kLog2e;
@@ -363,14 +387,10 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
     if (o_dma) {
       lds_barrier();
       const int orow = 32 * (wave & 1) + l32;
-      float part = 0.f;
 #pragma unroll
-      for (int ds = 0; ds < DS; ++ds) {
-        const frag of = lds_frag<T>(ring[NS - 1][wave >> 1] + tile_off<D>(orow, 2 * ds + g));
-#pragma unroll
-        for (int e = 0; e < 8; ++e) part = fmaf((float)of[e], (float)dof[ds][e], part);
-      }
-      finish_delta(part);
+      for (int ds = 0; ds < DS; ++ds)
+        add_chunk(ds, lds_frag<T>(ring[NS - 1][wave >> 1] + tile_off<D>(orow, 2 * ds + g)));
+      finish_delta(row_part());
 #pragma unroll
       for (int r = 0; r < 16; ++r) nd16[r] = -Dq;
     }
@@ -890,19 +910,22 @@ static hipError_t launch_dq16_t(const void* q, const void* k, const void* v, con
   const long long nblocks = (long long)p.nblk * p.B * p.H;
   p.wi_blocks_fastest = !p.causal;
   p.div_wi = p.wi_blocks_fastest ? work_item_div_blocks(p.nblk) : work_item_div((long long)p.B * p.H);
-  // Variants: block-causal (BLK) x delta fused in (FD, when p.o is set).
-  const auto go = [&](auto blk_c, auto fd_c) {
-    hipLaunchKernelGGL((attn_bwd16_dq_kernel<T, D, decltype(blk_c)::value, decltype(fd_c)::value>),
+  // Variants: block-causal (BLK) x delta fused in (FD, when p.o is set), gated or not.
+  const auto go = [&](auto blk_c, auto fd_c, auto gate_c) {
+    hipLaunchKernelGGL((attn_bwd16_dq_kernel<T, D, decltype(blk_c)::value, decltype(fd_c)::value,
+                                             decltype(gate_c)::value>),
                        dim3((unsigned)nblocks), dim3(256), 0, st, (const T*)q, (const T*)k,
                        (const T*)v, (const T*)dout, lse, delta, (T*)dq, p);
   };
   using yes = std::true_type;
   using no = std::false_type;
-  if (p.block > 1) {
-    if (p.o) go(yes{}, yes{}); else go(yes{}, no{});
-  } else {
-    if (p.o) go(no{}, yes{}); else go(no{}, no{});
-  }
+  const auto by_fd = [&](auto blk_c) {
+    if (p.o && p.gate) go(blk_c, yes{}, yes{});
+    else if (p.o) go(blk_c, yes{}, no{});
+    else go(blk_c, no{}, no{});
+  };
+  if (p.block > 1) by_fd(yes{});
+  else by_fd(no{});
   return hipGetLastError();
 }
 

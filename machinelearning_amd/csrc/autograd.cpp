@@ -139,11 +139,6 @@ struct Attn : torch::autograd::Function<Attn> {
       } else if (!gate.defined()) {
         check(mi_attn_bwd(ptr(q), ptr(k), ptr(v), ptr(o), ptr(dy), floats(lse), floats(dl),
                           floats(ws), ptr(dq), ptr(dk), ptr(dv), &s, st));
-      } else if (!dl.defined() && s.dtype != MI_F32) {
-        dz = at::empty_like(gate);
-        check(mi_attn_bwd_gated_direct(ptr(q), ptr(k), ptr(v), floats(gate), ptr(o), ptr(dy),
-                                       floats(lse), floats(ws), ptr(dq), ptr(dk), ptr(dv),
-                                       floats(dz), &s, st));
       } else {
         const Tensor dy_attn = at::empty_like(dy);   // sigmoid(gate) * dy, the kernels' input
         dz = at::empty_like(gate);

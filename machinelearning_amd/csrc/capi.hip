@@ -165,6 +165,7 @@ mi::AttnParams params(const mi_attn_shape* s) {
   p.kv_rs = (long long)s->Hkv * s->D;
   p.gate = nullptr;
   p.dgate = nullptr;
+  p.doe = nullptr;
   p.o = nullptr;
   p.dlse = nullptr;
   p.ws_out = nullptr;
@@ -359,15 +360,17 @@ int run_dkdv(const void* q, const void* k, const void* v, const void* dout, cons
                                        sink_part(delta, s), dk, dv, nullptr, p, stream));
 }
 
-// With `o` set (16-bit inputs, or float32 on the split-walk kernels), the dQ kernel also computes the delta
-// pass and writes both workspace planes (`delta`), from o and dlse.
+// With `o` set (16-bit inputs, or float32 on the split-walk kernels), the dQ kernel also
+// computes the delta pass and writes both workspace planes (`delta`), from o and dlse, and
+// with a gate (16-bit only) `doe` and dgate.
 int run_dq(const void* q, const void* k, const void* v, const void* dout, const float* lse,
            const float* delta, void* dq, const mi_attn_shape* s, hipStream_t stream,
            SinkPass sp, const void* o = nullptr, const float* dlse = nullptr,
-           const void* o_res = nullptr, const float* gate = nullptr, float* dgate = nullptr) {
+           const void* o_res = nullptr, const float* gate = nullptr, void* doe = nullptr,
+           float* dgate = nullptr) {
   if (!q || !k || !v || !dout || !lse || !delta || !dq) return MI_ERR_NULL;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(dout) || !aligned16(dq) ||
-      (o && !aligned16(o)))
+      (o && !aligned16(o)) || (doe && !aligned16(doe)))
     return MI_ERR_ALIGN;
   mi::AttnParams p = params(s);
   if (o) {
@@ -376,6 +379,7 @@ int run_dq(const void* q, const void* k, const void* v, const void* dout, const 
     p.ws_out = const_cast<float*>(delta);
     p.o_res = const_cast<void*>(o_res);
     p.gate = gate;
+    p.doe = doe;
     p.dgate = dgate;
   }
   const hipError_t e =
@@ -415,8 +419,9 @@ int mi_attn_bwd_dq(const void* q, const void* k, const void* v, const void* dout
 
 namespace {
 
-// The full backward; with a gate, stage 1 writes the gate-scaled output
-// gradient into dout_attn and the later passes read that instead of dout.
+// The full backward; with a gate, the delta pass (its own launch, or inside dQ)
+// writes the gate-scaled output gradient into dout_attn and the later passes
+// read that instead of dout.
 int run_bwd(const void* q, const void* k, const void* v, const float* gate, const void* o,
             const void* dout, const float* lse, const float* dlse, float* delta, void* dout_attn,
             void* dq, void* dk, void* dv, float* dgate, const mi_attn_shape* s,
@@ -428,15 +433,18 @@ int run_bwd(const void* q, const void* k, const void* v, const float* gate, cons
   if (o_res && !aligned16(o_res)) return MI_ERR_ALIGN;
   if (!q || !k || !v || !o || !dout || !lse || !delta || !dq || !dk || !dv) return MI_ERR_NULL;
   const mi::AttnParams p = params(s);
-  if (!gate && (s->dtype != MI_F32 || mi::f32_split_walk(p, s->H, true))) {
-    // No gate, and a dQ kernel that can: the dQ kernel computes the delta pass itself and runs
-    // first; dK/dV (and the sink pass) then read the planes it wrote.
+  const void* g = gate ? dout_attn : dout;
+  if (s->dtype != MI_F32 || (!gate && mi::f32_split_walk(p, s->H, true))) {
+    // A dQ kernel that can computes the delta pass itself and runs first; dK/dV
+    // (and the sink pass) then read the planes it wrote.
     if (!aligned16(o) || !aligned16(delta)) return MI_ERR_ALIGN;
     if (!mi::sink_bwd_fusable(p)) {
-      int r = run_dq(q, k, v, dout, lse, delta, dq, s, stream, SinkPass::kOwn, o, dlse, o_res);
+      int r = run_dq(q, k, v, dout, lse, delta, dq, s, stream, SinkPass::kOwn, o, dlse, o_res, gate,
+                     dout_attn, dgate);
       if (r) return r;
-      return run_dkdv(q, k, v, dout, lse, delta, dk, dv, s, stream, SinkPass::kOwn, allow_split);
+      return run_dkdv(q, k, v, g, lse, delta, dk, dv, s, stream, SinkPass::kOwn, allow_split);
     }
+    // Only float32 has separate sink passes, and its gated backward is the one below.
     int r = run_dq(q, k, v, dout, lse, delta, dq, s, stream, SinkPass::kNone, o, dlse, o_res);
     if (r) return r;
     r = run_dkdv(q, k, v, dout, lse, delta, dk, dv, s, stream, SinkPass::kNone, allow_split);
@@ -446,7 +454,6 @@ int run_bwd(const void* q, const void* k, const void* v, const float* gate, cons
   }
   int r = run_delta(o, dout, gate, lse, dlse, delta, dout_attn, dgate, s, stream);
   if (r) return r;
-  const void* g = gate ? dout_attn : dout;
   if (!mi::sink_bwd_fusable(p)) {
     r = run_dkdv(q, k, v, g, lse, delta, dk, dv, s, stream, SinkPass::kOwn, allow_split);
     if (r) return r;
@@ -542,23 +549,6 @@ int mi_attn_bwd_gated(const void* q, const void* k, const void* v, const float* 
   if (!gate || !dout_attn || !dgate) return MI_ERR_NULL;
   return run_bwd(q, k, v, gate, o, dout, lse, dlse, delta, dout_attn, dq, dk, dv, dgate, s,
                  stream);
-}
-
-int mi_attn_bwd_gated_direct(const void* q, const void* k, const void* v, const float* gate,
-                             const void* o, const void* dout, const float* lse, float* delta,
-                             void* dq, void* dk, void* dv, float* dgate, const mi_attn_shape* s,
-                             hipStream_t stream) {
-  const int st = validate(s);
-  if (st) return st;
-  if (s->dtype == MI_F32) return MI_ERR_DTYPE;
-  if (empty(s)) return MI_OK;
-  if (!q || !k || !v || !gate || !o || !dout || !lse || !delta || !dq || !dk || !dv || !dgate)
-    return MI_ERR_NULL;
-  if (!aligned16(o) || !aligned16(delta)) return MI_ERR_ALIGN;
-  const int r = run_dq(q, k, v, dout, lse, delta, dq, s, stream, SinkPass::kNone, o, nullptr, nullptr,
-                       gate, dgate);
-  if (r) return r;
-  return run_dkdv(q, k, v, dout, lse, delta, dk, dv, s, stream, SinkPass::kNone);
 }
 
 namespace {

@@ -324,13 +324,6 @@ def _bwd(do, dlse, q, k, v, o, lse, causal, window, sinks, scale, gate=None, blo
                                  do.data_ptr(), lse.data_ptr(),
                                  None if dlse is None else dlse.data_ptr(), delta.data_ptr(),
                                  dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), sp, _stream(q))
-        elif dlse is None and q.dtype in MMA_DTYPES:
-            dgate = torch.empty_like(gate)
-            st = lib.mi_attn_bwd_gated_direct(q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                              gate.data_ptr(), o.data_ptr(), do.data_ptr(),
-                                              lse.data_ptr(), delta.data_ptr(), dq.data_ptr(),
-                                              dk.data_ptr(), dv.data_ptr(), dgate.data_ptr(), sp,
-                                              _stream(q))
         else:
             do_attn = torch.empty_like(do)          # sigmoid(gate) * do, the kernels' input
             dgate = torch.empty_like(gate)

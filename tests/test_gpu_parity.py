@@ -1021,10 +1021,9 @@ def test_f32_full_chip_short_walks(B, T, D, window):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D,mode", [(32, "blocks"), (64, "window+sinks"), (64, "noncausal"),
                                     (128, "causal")])
-def test_gated_backward_without_dout_copy(dtype, D, mode):
-    """The gated backward that folds sigma into the planes: logits over the whole range
-    (sigma 1 down to underflow), at the plain bounds and finite; and an LSE gradient, which
-    takes the other route, adds to it."""
+def test_gated_backward_over_the_logit_range(dtype, D, mode):
+    """The gated backward with logits over the whole range (sigma 1 down to underflow),
+    at the plain bounds and finite; and an LSE gradient adds to it."""
     B, T, H, Hkv = 2, 150, 4, 2
     q, k, v, do = _rand(B, T, H, Hkv, D, dtype, seed=D)
     g = torch.Generator().manual_seed(D)
@@ -1044,9 +1043,9 @@ def test_gated_backward_without_dout_copy(dtype, D, mode):
     want = [o * sg[..., None], lw, *orc.backward(q, k, v, o, lw, dof, scale, causal, window,
                                                  sinks=sinks, block=block)]
     got = [t.detach().double().cpu().numpy() for t in (y, lse, *grads[:3])]
-    _compare(got, want, dtype, f"gated direct {mode} D{D} {dtype}")
+    _compare(got, want, dtype, f"gated range {mode} D{D} {dtype}")
     dz = (do.double().numpy() * o).sum(-1) * sg * (1 - sg)
-    _parity.check(f"gated direct {mode} D{D} {dtype}", "dgate", grads[3].double().cpu().numpy(), dz,
+    _parity.check(f"gated range {mode} D{D} {dtype}", "dgate", grads[3].double().cpu().numpy(), dz,
                   dtype)
     dl = torch.randn(B, H, T, generator=g)
     both = torch.autograd.grad((y, lse), xs[:3], (do.cuda(), dl.cuda()))
@@ -1054,3 +1053,84 @@ def test_gated_backward_without_dout_copy(dtype, D, mode):
                                       block=block, dlse=dl)]
     for n, a, b in zip(("dQ", "dK", "dV"), both, want[2:]):
         _parity.check(f"gated + dLSE {mode} D{D} {dtype}", n, a.double().cpu().numpy(), b, dtype)
+
+
+# One head per logit: open, and closed as far as sigma * dO stays a normal number of the
+# type (float16 with dO scaled as loss scaling does).
+CLOSED = {torch.float16: (0.0, -4.0, -6.0, -8.0, -10.0), torch.bfloat16: (0.0, -20.0, -60.0, -80.0)}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,D,causal", [(1030, 64, False), (1030, 32, True), (700, 128, False)])
+def test_gated_backward_of_closed_heads(dtype, T, D, causal):
+    """A head whose gate is closed everywhere: its gradients against its own norm.
+
+    Each operand of dV = P^T (sigma dO) and the result are rounded once (u each), so
+    |err| <= 3 u |dV| row by row where they are normal numbers; 4 u leaves a quarter for
+    float16's P below 2^-14. dQ and dK have the roundings of dS, of the operand and
+    of the result, and that of the stored output inside Delta: 4 u (bfloat16 only:
+    float16's sigma P dP leaves the normal range on both routes).
+    """
+    zs = CLOSED[dtype]
+    B, H = 1, len(zs)
+    q, k, v, do = _rand(B, T, H, H, D, dtype, seed=T, do_std=1.0 if dtype == torch.bfloat16 else 256.0)
+    g = torch.Generator().manual_seed(T)
+    z = torch.tensor(zs).expand(B, T, H) + 0.5 * torch.randn(B, T, H, generator=g)
+    scale = 1.0 / math.sqrt(D)
+    got = _gpu_gated(q, k, v, do, z, causal, 0, scale)
+    o, lw = orc.forward(q, k, v, scale, causal, 0)
+    dof = do.double().numpy() / (1 + np.exp(-z.double().numpy()))[..., None]
+    want = orc.backward(q, k, v, o, lw, dof, scale, causal, 0)
+    u = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for h, zh in enumerate(zs):
+        for i, n in enumerate(("dQ", "dK", "dV")):
+            a, b = got[2 + i][:, :, h], want[i][:, :, h]
+            rel = float(np.linalg.norm(a - b) / np.linalg.norm(b))
+            print(f"closed head {dtype} T{T} D{D} logit {zh}: {n} rel {rel:.2e}", flush=True)
+            if n == "dV" or dtype == torch.bfloat16:
+                assert rel <= 4 * u, (n, zh, rel)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("mode", ["causal", "noncausal", "window+sinks", "blocks", "gqa split"])
+@pytest.mark.parametrize("with_dlse", [False, True], ids=["", "dlse"])
+def test_gated_delta_inside_dq_has_the_bits_of_the_passes(dtype, D, mode, with_dlse):
+    """mi_attn_bwd_gated (16-bit: the delta pass inside dQ, O by LDS-DMA or direct) ==
+    delta_gated, dkdv and dq one by one, bit for bit, on ragged rows: gradients, the gate's
+    gradient, sigma * dO and both planes."""
+    import ctypes
+    from machinelearning_amd import _capi
+    lib = _capi.load()
+    B, T, H, Hkv = 2, 147, 6, 2 if mode == "gqa split" else 6
+    causal = mode != "noncausal"
+    window, sinks = (24, 3) if "sinks" in mode else (0, 0)
+    q, k, v, do = (t.cuda() for t in _rand(B, T, H, Hkv, D, dtype, seed=D))
+    z = (3 * _gate_logits(B, T, H, D)).cuda()
+    dl = torch.randn(B, H, T, generator=torch.Generator().manual_seed(D)).cuda()
+    shp = _capi.shape(B, T, H, Hkv, D, causal, window, D ** -0.5,
+                      _capi.MI_BF16 if dtype == torch.bfloat16 else _capi.MI_F16, sinks,
+                      20 if mode == "blocks" else 0)
+    sp, st = ctypes.byref(shp), torch.cuda.current_stream().cuda_stream
+    P = lambda t: t.data_ptr()
+    dlp = P(dl) if with_dlse else None
+    o, lse = torch.empty_like(q), torch.empty(B, H, T, device="cuda")
+    assert lib.mi_attn_fwd_gated(P(q), P(k), P(v), P(z), P(o), P(lse), sp, st) == 0
+    outs = []
+    for full in (True, False):
+        ws = torch.empty(_capi.workspace_floats(shp), device="cuda")
+        doa, dz = torch.empty_like(do), torch.empty_like(z)
+        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+        if full:
+            assert lib.mi_attn_bwd_gated(P(q), P(k), P(v), P(z), P(o), P(do), P(lse), dlp,
+                                         P(ws), P(doa), P(dq), P(dk), P(dv), P(dz), sp, st) == 0
+        else:
+            assert lib.mi_attn_bwd_delta_gated(P(o), P(do), P(z), P(lse), dlp, P(ws), P(doa),
+                                               P(dz), sp, st) == 0
+            assert lib.mi_attn_bwd_dkdv(P(q), P(k), P(v), P(doa), P(lse), P(ws), P(dk), P(dv),
+                                        sp, st) == 0
+            assert lib.mi_attn_bwd_dq(P(q), P(k), P(v), P(doa), P(lse), P(ws), P(dq), sp, st) == 0
+        torch.cuda.synchronize()
+        outs.append([dq, dk, dv, dz, doa, ws[:2 * B * H * T]])
+    for n, a, b in zip(("dQ", "dK", "dV", "dgate", "sigma dO", "planes"), *outs):
+        assert torch.equal(a, b), n
