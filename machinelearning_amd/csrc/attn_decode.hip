@@ -215,14 +215,16 @@ struct Dec16 {
 // one BN-key block held in LDS as natural K / V tiles (swizzled chunks, the
 // forward kernel's layout and fragment maps) plus, with a window, the keys'
 // positions.
-// HL: P enters the PV product as two 16-bit terms, its rounding and the
-// rounding of the residual (~16 significant bits), for steps of a few rows,
-// whose probabilities the VALU kernel holds in fp32; the second MFMA is free
-// there (the step waits for K and V).
-template <typename T, int D, bool SWA, bool HL = false>
+// P32: P enters the PV product in fp32's 24 bits, as three 16-bit terms (each the
+// rounding of what the ones before leave), for steps of a few rows, whose
+// probabilities the VALU kernel holds in fp32; the extra MFMAs are free there
+// (the step waits for K and V). float16 terms are of 2^14 P (P <= 1), so that they
+// stay normal down to P = 2^-28; `unscale` takes the factor, exact, out of O.
+template <typename T, int D, bool SWA, bool P32 = false>
 struct Dec16Rows {
   using C = Dec16<D>;
   using M = Mfma32<T>;
+  static constexpr float kPScale = P32 && std::is_same_v<T, _Float16> ? 16384.f : 1.f;
   using frag = typename M::frag;
   static constexpr int BN = C::BN, MT = C::MT, DS = C::DS, DT = C::DT;
   frag qf[DS];
@@ -343,17 +345,38 @@ struct Dec16Rows {
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        const frag pb = pack_frag<T>(s[mt], ks * 8);
-        frag pl;
-        if constexpr (HL) pl = lo_frag<T>(s[mt], ks * 8, pb);
+        constexpr int NP = P32 ? 3 : 1;
+        frag pb[NP];
+        if constexpr (P32) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            float x = s[mt][ks * 8 + e] * kPScale;
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+              pb[i][e] = (T)x;
+              x -= (float)pb[i][e];
+            }
+          }
+        } else {
+          pb[0] = pack_frag<T>(s[mt], ks * 8);
+        }
         const int roff = (32 * mt + 16 * ks) * D * 2;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           const frag vt = lds_frag_tr<T>(sV + vaddr[dt][0] + roff, sV + vaddr[dt][1] + roff);
-          oacc[dt] = M::mma(vt, pb, oacc[dt]);
-          if constexpr (HL) oacc[dt] = M::mma(vt, pl, oacc[dt]);
+#pragma unroll
+          for (int i = NP - 1; i >= 0; --i) oacc[dt] = M::mma(vt, pb[i], oacc[dt]);
         }
       }
+  }
+
+  __device__ __forceinline__ void unscale() {
+    if constexpr (kPScale != 1.f) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) oacc[dt][i] *= 1.f / kPScale;
+    }
   }
 };
 
@@ -404,7 +427,7 @@ struct Dec16Stage {
 // At most 32 query rows per kv head: each wave streams its own blocks (every
 // WS-th of the split) through its private LDS tile, with no workgroup barrier
 // in the loop, and the waves merge at the end.
-template <typename T, int D, bool SWA, bool HL>
+template <typename T, int D, bool SWA, bool P32>
 __global__ void __launch_bounds__(64 * Dec16<D>::WS)
 attn_decode16_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const T* __restrict__ Vc,
                      const T* __restrict__ Kn, const T* __restrict__ Vn, T* __restrict__ O,
@@ -429,7 +452,7 @@ attn_decode16_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const T*
   char* sV = tiles[wave] + C::TILE;
   int* sP = reinterpret_cast<int*>(tiles[wave] + 2 * C::TILE);
 
-  Dec16Rows<T, D, SWA, HL> st;
+  Dec16Rows<T, D, SWA, P32> st;
   st.init(p, Q, b, kvh, tile, lane);
   const DecRows rows = dec_rows<T>(p, Kc, Vc, Kn, Vn, b, kvh);
   Dec16Stage<T, D, 64> stage;
@@ -451,6 +474,7 @@ attn_decode16_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const T*
   // Merge the waves. Each wave writes its rows' (m, l) and O into its own
   // LDS (its tile bytes: 32 * D * 4 <= 2 * TILE), then all threads combine.
   const float l_tot = halves_sum(st.l_run);
+  st.unscale();
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   float* ob = reinterpret_cast<float*>(tiles[wave]);
 #pragma unroll
@@ -930,17 +954,19 @@ static void dec_geometry(DecParams& p) {
 // products and converted keys hold a lone VALU workgroup back, while an MFMA's
 // padded columns cost nothing; but its eight waves' tiles fill a CU's LDS (half
 // of it at D = 32), so it wins where the workgroups are one round of the chip,
-// and the VALU kernel's smaller ones beyond. One step, us, VALU -> MFMA (grid =
-// workgroups):
-//   grid 8    B1 H32/8 L1000 D128   30.3 -> 16.4    grid 320  B10 H32/8 L2048 D128  24.1 -> 27.9
-//   grid 128  B4 H24/8 L2048 D128   22.4 -> 15.4    grid 512  B8 H32/8 L4096 D128   30.5 -> 33.9
-//   grid 256  B4 H16/8 L4096 D128   23.9 -> 20.3    grid 512  B16 H16/8 L4096 D64   30.2 -> 32.5
-//   grid 192  B16 T2 H12 L1024 D64  19.8 -> 12.0    grid 640  B80 H32/8 L800 D64    28.5 -> 34.2
-//   grid 256  B8 H32/8 L4096 D64    24.2 -> 18.4    grid 512  B16 H16/8 L8192 D32   30.6 -> 28.6
-template <int D>
+// and the VALU kernel's smaller ones beyond; under 256 keys its waves have no
+// blocks to overlap and the merge of eight shows (7.1 -> 7.7 us at 30 keys, D
+// 128). One step, us, VALU -> MFMA with P in three terms, bf16 (f16 up to 2 us
+// more than bf16; grid = workgroups):
+//   grid 8    B1 H32/8 L1000 D128   30.2 -> 17.8    grid 256  B32 H32/8 L500 D64    11.2 -> 9.1
+//   grid 128  B4 H24/8 L2048 D128   21.8 -> 16.0    grid 320  B40 H32/8 L2000 D32   23.9 -> 24.4
+//   grid 256  B4 H16/8 L4096 D128   23.5 -> 20.8    grid 512  B64 H32/8 L1000 D32   16.1 -> 17.9
+//   grid 192  B16 T2 H12 L1024 D64  19.8 -> 13.1    grid 320  B10 H32/8 L2048 D128  24.1 -> 27.9
+//   grid 256  B8 H32/8 L4096 D64    23.5 -> 20.0    grid 512  B16 H16/8 L4096 D64   30.2 -> 32.5
+// (the last two with P in two terms).
 static bool dec_small_mfma(const DecParams& p) {
   const long long grid = (long long)p.B * p.Hkv * p.nsplit;
-  return p.R >= 2 && p.R <= kDecValuRows && grid <= (D <= 32 ? 512 : 256);
+  return p.R >= 2 && p.R <= kDecValuRows && p.Lk >= 256 && grid <= 256;
 }
 
 template <typename T, int D, int RT>
@@ -974,7 +1000,7 @@ static hipError_t launch_decode_t(const void* q, const void* kc, const void* vc,
       break;
     case kDecValuRows:
       if constexpr (sizeof(T) == 2) {
-        if (dec_small_mfma<D>(p)) {
+        if (dec_small_mfma(p)) {
           DecParams m = p;   // the same key ranges in the MFMA kernel's blocks
           static_assert(DecV<T, D, kDecValuRows>::BN % Dec16<D>::BN == 0, "whole blocks");
           m.bps = p.bps * (DecV<T, D, kDecValuRows>::BN / Dec16<D>::BN);

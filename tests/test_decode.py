@@ -546,11 +546,12 @@ def test_window_commit_equals_boolean_indexing(dtype, Lc, T, window, sinks, evic
     assert torch.equal(cache["k"], kf[:, :, live]) and torch.equal(cache["v"], vf[:, :, live])
 
 
-# (B, T, cached, H, Hkv): two to four query rows per kv head, on both sides of the grid
-# where the MFMA kernel takes them (one round of workgroups), split and unsplit, key
-# counts around its 32 / 64-key blocks.
+# (B, T, cached, H, Hkv): two to four query rows per kv head, on both sides of the key
+# count (256) and of the grid (one round of workgroups) from which on the MFMA kernel
+# takes them, split and unsplit, key counts around its 32 / 64-key blocks.
 SMALL_ROWS = [(1, 1, 31, 4, 2), (1, 2, 64, 3, 3), (2, 1, 700, 6, 2), (1, 4, 65, 2, 2),
-              (1, 1, 9000, 8, 2), (3, 2, 2100, 4, 2), (70, 1, 40, 32, 8)]
+              (1, 1, 9000, 8, 2), (3, 2, 2100, 4, 2), (70, 1, 40, 32, 8), (1, 1, 254, 4, 2),
+              (1, 1, 255, 4, 2), (1, 2, 286, 3, 3), (2, 4, 319, 2, 2), (40, 1, 256, 16, 8)]
 
 
 @pytest.mark.gpu
@@ -591,3 +592,46 @@ def test_decode_more_than_32_rows(dtype, D, shape, causal):
     k, v = (g.standard_normal((B, T, Hkv, D)) for _ in range(2))
     cache = {n: g.standard_normal((B, Hkv, Lc, D)) for n in "kv"}
     _step(q, k, v, cache, dtype, causal, tag=f"decode many rows {dtype} D{D} {shape} {causal}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES[1:], ids=lambda d: str(d).replace("torch.", ""))
+@pytest.mark.parametrize("keys", ["few", "many small"])
+def test_decode_two_to_four_rows_hold_p_in_fp32(dtype, keys):
+    """The rounding of the output aside, P and the sums are fp32's: keys whose scores are
+    exact products. "few" makes P's own rounding visible (seven keys near P = 1, 0 on the
+    others), "many small" float16's range (one key at P = 1 with V = 0, 1999 near 1e-4).
+
+    |err| <= half an ulp of the output + 1e-6 sum P |V|: exp2's argument, at most 14, is
+    rounded to 2^-21 and its scale factor to 2^-25 (5e-7 and 3e-7 of P), the rest is ulps of
+    the exponential and of the sums.
+    """
+    from machinelearning_amd.decode import attn_cached
+    B, H, Hkv, D = 16, 32, 8, 32
+    g = torch.Generator(device="cuda").manual_seed(5)
+    L = 300 if keys == "few" else 1999
+    lo, hi = (-1.0, 0.0) if keys == "few" else (-9.5, -8.5)
+    t = lo + (hi - lo) * torch.rand(B, Hkv, L + 1, generator=g, device="cuda")
+    t[:, :, -1] = 0
+    if keys == "few":
+        t[:, :, 6:-1] = -200
+    k = torch.zeros(B, Hkv, L + 1, D, device="cuda")
+    k[..., 0] = t
+    v = torch.randn(B, Hkv, L + 1, D, generator=g, device="cuda")
+    if keys != "few":
+        v[:, :, -1] = 0
+    q = torch.zeros(B, 1, H, D, device="cuda")
+    q[..., 0] = 1.0 - torch.arange(H, device="cuda") % 4 / 8
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    cache = {"k": k[:, :, :L].contiguous(), "v": v[:, :, :L].contiguous()}
+    with torch.no_grad():
+        y = attn_cached(q, k[:, :, L:].transpose(1, 2).contiguous(),
+                        v[:, :, L:].transpose(1, 2).contiguous(), cache, False, True, scale=1.0)
+    s = q.double().view(B, Hkv, H // Hkv, D)[..., :1] * k.double()[:, :, None, :, 0]
+    p = torch.softmax(s, -1)                                           # B Hkv rep keys
+    ref = torch.stack([(p[:, :, r, :, None] * v.double()).sum(2) for r in range(H // Hkv)], 2)
+    mag = torch.stack([(p[:, :, r, :, None] * v.double().abs()).sum(2) for r in range(H // Hkv)], 2)
+    err = (y.double().view(ref.shape) - ref).abs().cpu().numpy()
+    tol = _parity.half_ulp(ref.cpu().numpy(), dtype) + 1e-6 * mag.cpu().numpy()
+    print(f"decode P fp32 {dtype} {keys}: worst err/tol {(err / tol).max():.3f}", flush=True)
+    assert (err <= tol).all(), (int((err > tol).sum()), err.size)
