@@ -501,28 +501,25 @@ attn_decode16_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const T*
 // (batch, kv head) and share every key block, staged once per workgroup
 // into LDS. (Per-wave streaming would read the keys once per 32-row tile.)
 // Bound by each wave's serial chain per step (LDS reads, MFMAs, max, exp,
-// MFMAs), with one or two waves per SIMD to hide it: without a window a step
-// takes two blocks, brought by LDS-DMA during the step before. Against one
-// block per step, double-buffered through registers (as still with a window,
-// whose visibility depends on each key's position), results the same bit for
-// bit: [8, 16, 32 / 8, 64] on 4096 keys 24.9 -> 23.2 us, [4, 64, 8 / 8, 64] on
-// 2000 24.0 -> 22.3, [4, 16, 12 / 4, 128] on 1500 28.5 -> 26.3, [2, 300, 8 / 4,
-// 128] on none 15.1 -> 14.3; [8, 32, 32 / 8, 128] on 4096, two workgroups on
-// every CU, stays at 41. LDS-DMA alone, one block per step: 23.9, 23.5, 27.4
-// and 16.5. One maximum for both blocks would give 22.3, 21.6 and 24.6, but P
-// is then exactly 1 less often, and the error grows by 0.5%.
+// MFMAs), with one or two waves per SIMD to hide it. Two ways to bring blocks, with
+// the same bits: one block per step, double-buffered through registers; or (DMA, no
+// window: a window's visibility depends on each key's position) two per step,
+// brought by LDS-DMA during the step before, in twice the LDS. dec_dma says when.
+// (One maximum for both blocks of a step would be another 4% faster, but P is
+// then exactly 1 less often, and the error grows by 0.5%.)
 // Each wave then writes its own rows: the output, or its split partial.
-template <typename T, int D, bool SWA>
+template <typename T, int D, bool SWA, bool DMA>
 __global__ void __launch_bounds__(256)
 attn_decode16_wg_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const T* __restrict__ Vc,
                         const T* __restrict__ Kn, const T* __restrict__ Vn, T* __restrict__ O,
                         float* __restrict__ LSE, float* __restrict__ ws, DecParams p) {
   using C = Dec16<D>;
   constexpr int W = C::W, BN = C::BN, DT = C::DT;
-  // With a window a double buffer of K tile, V tile and the keys' positions;
-  // else a ring of four K tiles, then of four V tiles.
-  constexpr int NS = SWA ? 2 : 4;
-  __shared__ __attribute__((aligned(1024))) char tiles[NS][2 * C::TILE + (SWA ? 256 : 0)];
+  static_assert(!(SWA && DMA), "a window's blocks come through registers");
+  // A double buffer of K tile, V tile and (with a window) the keys' positions; with DMA
+  // a ring of four K tiles, then of four V tiles.
+  constexpr int NS = DMA ? 4 : 2;
+  __shared__ __attribute__((aligned(1024))) char tiles[NS][2 * C::TILE + (DMA ? 0 : 256)];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ngrp = (p.ntiles + W - 1) / W;
@@ -539,7 +536,7 @@ attn_decode16_wg_kernel(const T* __restrict__ Q, const T* __restrict__ Kc, const
 
   const int nblk = (p.Lk + BN - 1) / BN;
   const int blk0 = split * p.bps, blk1 = min(nblk, blk0 + p.bps);
-  if constexpr (SWA) {
+  if constexpr (!DMA) {
     if (blk0 < blk1) stage.load(p, rows, blk0, tid, SWA);
     for (int blk = blk0; blk < blk1; ++blk) {
       // Buffer (blk & 1) was last read in block blk - 2; every wave passed the
@@ -969,6 +966,38 @@ static bool dec_small_mfma(const DecParams& p) {
   return p.R >= 2 && p.R <= kDecValuRows && p.Lk >= 256 && grid <= 256;
 }
 
+// More than 32 16-bit rows per kv head, no window: whether the blocks come by
+// LDS-DMA, two a step. It takes the wave's step off the load's path, where the
+// chip has at most a workgroup per CU (two on long walks); its ring halves the
+// workgroups a CU holds (not at D = 128, whose registers allow two anyway), and keys of the active block go through registers with
+// nothing to hide them (from an empty cache they are DMA too), so it loses on
+// larger grids and where the block is a good part of a split. One step, us, through
+// registers -> DMA, bf16 (grid = workgroups, bps = blocks per split, past = blocks
+// that reach past the cache):
+//   D64   grid 96   bps 17 past 1   22.9 -> 20.8    D128  grid 192  bps 17 past 2   23.1 -> 22.0
+//   D64   grid 12   bps 9  past 1   13.0 -> 12.1    D128  grid 512  bps 65 past 2    116 -> 112
+//   D64   grid 512  bps 33 past 1   71.1 -> 67.8    D128  grid 256  bps 11 past 5   17.8 -> 20.0
+//   D64   grid 512  bps 17 past 2   36.6 -> 38.6    D128  grid 512  bps 18 past 2   33.8 -> 35.4
+//   D64   grid 768  bps 4  past 1   14.9 -> 19.2    D128  grid 1024 bps 34 past 33   105 -> 120
+//   D64   grid 256  bps 17 past 17  24.5 -> 26.2    D32   grid 512  bps 33 past 1   51.2 -> 50.0
+//   D64   grid 384  bps 16 empty    31.7 -> 30.8    D32   grid 192  bps 17 past 2   16.0 -> 16.4
+//   D64   grid 768  bps 16 empty    48.5 -> 52.6    D128  grid 2048 bps 32 empty     196 -> 181
+//   D64   grid 512  bps 80 past 16   123 -> 117     D128  grid 608  bps 69 past 10   172 -> 164
+template <typename T, int D>
+static bool dec_dma(const DecParams& p) {
+  const int nblk = (p.Lk + Dec16<D>::BN - 1) / Dec16<D>::BN;
+  const long long grid = (long long)p.B * p.Hkv * dec_groups<T, D>(p) * p.nsplit;
+  if (p.Lc == 0) {
+    if (grid <= 256) return D < 128 || p.bps >= 4;
+    if (grid <= 512) return p.bps >= 5;
+    return D == 128 && p.bps >= 10;
+  }
+  const int past = nblk - p.Lc / Dec16<D>::BN;
+  if (D >= 64 && grid <= 256) return past * (D == 64 ? 2 : grid <= 64 ? 4 : 8) <= p.bps;
+  if (p.bps >= 64) return past * 4 <= p.bps && (D == 128 || grid <= 512);
+  return D <= 64 && p.bps >= (D == 64 ? 16 : 32) && past * 16 <= p.bps && grid <= 512;
+}
+
 template <typename T, int D, int RT>
 static void launch_valu(dim3 grid, bool swa, const T* Q, const T* Kc, const T* Vc, const T* Kn,
                         const T* Vn, T* out, float* lse, float* ws, const DecParams& p,
@@ -1019,11 +1048,14 @@ static hipError_t launch_decode_t(const void* q, const void* kc, const void* vc,
       if constexpr (sizeof(T) == 2) {
         const bool shared = p.R > Dec16<D>::RT;
         if (shared && swa)
-          hipLaunchKernelGGL((attn_decode16_wg_kernel<T, D, true>), grid, dim3(256), 0, st, Q, Kc,
-                             Vc, Kn, Vn, (T*)out, lse, ws, p);
+          hipLaunchKernelGGL((attn_decode16_wg_kernel<T, D, true, false>), grid, dim3(256), 0, st, Q,
+                             Kc, Vc, Kn, Vn, (T*)out, lse, ws, p);
+        else if (shared && dec_dma<T, D>(p))
+          hipLaunchKernelGGL((attn_decode16_wg_kernel<T, D, false, true>), grid, dim3(256), 0, st, Q,
+                             Kc, Vc, Kn, Vn, (T*)out, lse, ws, p);
         else if (shared)
-          hipLaunchKernelGGL((attn_decode16_wg_kernel<T, D, false>), grid, dim3(256), 0, st, Q, Kc,
-                             Vc, Kn, Vn, (T*)out, lse, ws, p);
+          hipLaunchKernelGGL((attn_decode16_wg_kernel<T, D, false, false>), grid, dim3(256), 0, st, Q,
+                             Kc, Vc, Kn, Vn, (T*)out, lse, ws, p);
         else if (swa)
           hipLaunchKernelGGL((attn_decode16_kernel<T, D, true, false>), grid, dim3(64 * Dec16<D>::WS), 0, st, Q, Kc, Vc,
                              Kn, Vn, (T*)out, lse, ws, p);

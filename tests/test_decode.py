@@ -573,11 +573,13 @@ def test_decode_two_to_four_rows(dtype, D, shape, mode):
           tag=f"decode rows {dtype} D{D} {shape} {mode}")
 
 
-# (B, T, cached, H, Hkv): more than 32 query rows per kv head, which share blocks staged
-# two at a time: an empty cache, a last pair of one block, one block with keys of both
-# the cache and the step, a cache that ends on a block, splits.
+# (B, T, cached, H, Hkv): more than 32 query rows per kv head, which share staged blocks,
+# one or two at a time: an empty cache, a last pair of one block, one block with keys of
+# both the cache and the step, a cache that ends on a block, splits, more workgroups
+# than the chip holds at once, a block longer than its cache.
 MANY_ROWS = [(1, 33, 0, 2, 2), (2, 70, 0, 4, 2), (1, 40, 1, 3, 3), (2, 17, 64, 8, 4),
-             (1, 34, 127, 2, 1), (1, 64, 130, 4, 2), (1, 9, 5001, 8, 2), (3, 33, 160, 2, 2)]
+             (1, 34, 127, 2, 1), (1, 64, 130, 4, 2), (1, 9, 5001, 8, 2), (3, 33, 160, 2, 2), (140, 33, 70, 4, 4),
+             (140, 34, 0, 4, 4), (2, 150, 35, 4, 2)]
 
 
 @pytest.mark.gpu
