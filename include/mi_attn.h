@@ -113,6 +113,11 @@ typedef struct {
  * (nanolab/csrc/flash_attn_cuda.cu:1628-1650). */
 MI_API int mi_attn_check(const mi_attn_shape* s);
 
+/* Which kernels a valid float32 call runs, by its shape: 1 where the forward (pass 0), dQ (1)
+ * or dK/dV (2) takes the 32-row kernels whose waves split the walk, 0 where the 128-row
+ * ones (and for every other call). Both compute in float32 and agree to its rounding. */
+MI_API int mi_attn_f32_split(const mi_attn_shape* s, int pass);
+
 /* Size in floats of the backward workspace `delta` for shape `s`: 2*B*H*S,
  * plus, for float32 with sinks that some query sees beyond its window span,
  * the sink pass's partial sums (16-bit kernels visit the sinks themselves),

@@ -82,6 +82,7 @@ _DSHAPE = ctypes.POINTER(MiDecodeShape)
 # name -> (restype, argtypes); the exported surface of include/mi_attn.h.
 SIGNATURES = {
     "mi_attn_check": (ctypes.c_int, [_SHAPE]),
+    "mi_attn_f32_split": (ctypes.c_int, [_SHAPE, ctypes.c_int]),
     "mi_attn_bwd_workspace": (ctypes.c_int, [_SHAPE, ctypes.POINTER(ctypes.c_longlong)]),
     "mi_attn_fwd": (ctypes.c_int, [_P, _P, _P, _P, _P, _SHAPE, _P]),
     "mi_attn_bwd": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _SHAPE, _P]),

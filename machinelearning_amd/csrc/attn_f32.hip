@@ -344,8 +344,7 @@ attn_f32_dkdv_kernel(const float* __restrict__ Q, const float* __restrict__ K,
   const Buf deltas = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(Delta), 0, (int)((long long)p.B * p.H * p.S * 4), 0x00020000);
   // The next tile's rows are loaded under this tile's products where the
-  // registers allow it (D <= 64); at D = 128 (1.3x the register file) at the
-  // tile's start.
+  // registers allow it (D = 32), else at the tile's start.
   constexpr bool AHEAD = D <= 32;
   // Iteration it: head hkv * group + it / ntq, query tile tq_begin + it % ntq.
   int gh = 0, tq = wave;
@@ -460,32 +459,83 @@ hipError_t f32_dispatch(int D, bool blk, F&& f) {
 
 }  // namespace
 
-// Whether a float32 launch of `heads` (query heads; kv heads for dK/dV) takes
-// these kernels. Against the 128-row kernels (fwd / bwd us at D = 64, causal,
-// before -> after; `grid` counts their workgroups, `walk` the rows of the other
-// side a row can see):
-//   grid 32,   walk 256  (B4 H4)            28.7 -> 8.7      95.8 -> 28.4
-//   grid 192,  walk 1024 (B2 H12)           95.4 -> 40.3    319 -> 141
-//   grid 768,  walk 1024 (B8 H12)          157.6 -> 125.5   507 -> 467
-//   grid 1024, walk 4096 (B2 H16)            697 -> 555    2200 -> 1931
-//   grid 768,  walk 256  (B32 H12)          68.5 -> 54.8    228 -> 218
-//   grid 1536, walk 1024 (B16 H12)           282 -> 259     961 -> 971
-//   grid 2048, walk 287  (SWA(256), S 4096)  256 -> 213     833 -> 861
-//   grid 768,  walk 128  (B64 H12)          44.4 -> 40.8    156 -> 172
-//   grid 768,  walk 100  (B64 H12 D128)     91.8 -> 96.5    329 -> 356
-// The split costs a merge and gives up the tiles shared by four waves, so a
-// short walk on a full chip stays with the others, and so does a backward of
-// middling walk once the chip is full six times over. Offsets inside a head
-// and the row vectors are 32-bit here (S <= 2 GiB of rows); larger tensors
-// stay with the others too.
-bool f32_split_walk(const AttnParams& p, int heads, bool backward) {
+// Modelled time of a launch here over that on the 128-row kernels: walk rows that the
+// busiest of 256 CUs passes, whole workgroups to a CU (a causal launch's last ones
+// are its shortest). Four waves of a 128-row workgroup each walk all of it, in
+// 64-row tiles; here they share it in 32-row tiles.
+static double split_share(const AttnParams& p, int heads) {
+  const auto up = [](long long a, long long b) { return (a + b - 1) / b; };
+  const long long bh = (long long)p.B * heads, n128 = up(p.S, 128), n32 = up(p.S, 32);
+  if (p.window > 0 && p.window < p.S - 31) {
+    const long long tiled = up(p.window + 127LL, 64) * 64 + 32, split = up(up(p.window + 31LL, 32) + 1, 4) * 32;
+    return (double)(up(n32 * bh, 256) * split) / (double)(up(n128 * bh, 256) * tiled);
+  }
+  const long long all = up(p.S, 64) * 64, each = up(n32, 4) * 32;
+  if (!p.causal) return (double)(up(n32 * bh, 256) * each) / (double)(up(n128 * bh, 256) * all);
+  const long long m = n32 / 4, tiled = 64 * n128 * (n128 - 1) + all,
+                  split = 32 * (2 * m * (m + 1) + (n32 % 4) * (m + 1));
+  const long long t = up(bh * tiled, 256 * 128) * 128, u = up(bh * split, 256 * 32) * 32;
+  return (double)(u > each ? u : each) / (double)(t > all ? t : all);
+}
+
+// Whether a float32 launch of `heads` (query heads; kv heads for dK/dV) takes these
+// kernels. Two things decide (`grid` counts the 128-row kernels' workgroups, `walk` the
+// rows of the other side a row can see). What the split saves: few workgroups, or rounds of
+// them that end half empty, which split_share models. What it costs: a merge, the
+// tiles that four waves no longer share (so more L2 traffic), and at D >= 64 one or
+// two waves per SIMD (and 4 / 15 spilled registers in dQ / dK/dV at D = 64): little on a
+// long walk, 10-25% on one of 100-250 rows of a chip that is full either way. The
+// limits are measured over 2100 shapes, each pass and D: none taken is over 5%
+// slower, three over 2.5%. 128-row kernels -> these, fwd / bwd us:
+//   causal   D64  grid 32    S256    28.7 -> 8.7     95.8 -> 28.4
+//            D64  grid 768   S1024    158 -> 126      507 -> 470
+//            D64  grid 504   S256    (causal bwd limit)   137 <- 151
+//            D128 grid 288   S1024    182 -> 119      606 -> 416
+//            D128 grid 1488  S256     271 <- 276      984 <- 1017
+//            D128 grid 3072  S2048   2357 -> 2228    7995 <- 8691
+//            D32  grid 768   S1024   86.8 -> 64.6     291 -> 237
+//   full     D64  grid 960   S1024    324 -> 277     1066 -> 976
+//            D64  grid 3000  S128     164 <- 189      609 <- (grid)
+//            D64  grid 1488  S256     142 -> 140      488 <- 557
+//            D128 grid 264   S256     109 -> 79       370 -> 266
+//            D128 grid 252   S128    36.5 <- 45.1     129 <- 143
+//            D32  grid 1488  S256    (fwd limit)      239 <- 265
+//   window   D64  grid 2048  256, S4096  254 -> 215   843 <- 861
+//            D128 grid 288   64, S3000  (0.52 of the time)
+// Offsets inside a head and the row vectors are 32-bit here (S <= 2 GiB of rows); larger
+// tensors stay with the others too.
+bool f32_split_walk(const AttnParams& p, int D, int heads, bool backward) {
   const long long row_bytes = 4LL * (p.q_rs > p.kv_rs ? p.q_rs : p.kv_rs);
   if ((p.S + 32LL) * row_bytes > 0x7fffffffLL) return false;
   if (4LL * (p.S + 32LL) * p.B * p.H > 0x7fffffffLL) return false;
   const long long grid = (p.S + 127LL) / 128 * p.B * heads;
-  const int walk = p.window > 0 && p.window < p.S - 31 ? p.window + 31 : p.S;
-  if (!backward) return grid < 512 || walk >= 128;
-  return grid < 512 || (grid < 1536 && walk >= 256) || walk >= 2048;
+  const long long walk = p.window > 0 && p.window < p.S - 31 ? p.window + 31LL : p.S;
+  if (grid >= 512) {
+    if (!backward ? walk < 128 : walk < 256 || (grid >= 1536 && walk < 2048)) return false;
+  }
+  if (walk <= 64) return true;
+  const long long rows = walk * (p.H / heads);   // dK/dV walks every query head of the group
+  // Walks of one full 128-row workgroup and at most half of another.
+  const bool half = walk > 128 && walk <= 192;
+  const bool few = grid <= 448 && rows > 128;
+  double limit = 9.0;
+  if (!p.causal && backward) {
+    if (D == 32 && (grid <= 256 || half)) limit = 9.0;
+    else if (D == 64 && grid <= 256 && rows >= 384 && rows <= 512) limit = 1.01;
+    else if (rows <= 128) limit = 0.7;
+    else if (rows <= 256) limit = D == 32 ? 0.89 : 0.8;
+    else if (rows <= (D == 128 ? 1024 : 512)) limit = 0.98;
+  } else if (!p.causal) {
+    if (D == 128) limit = walk <= 256 ? 0.85 : walk <= 400 ? 0.98 : 9.0;
+    else if (walk <= 128) limit = grid <= 256 ? 1.01 : 0.9;
+    else if (walk <= 256 && !half) limit = 0.95;
+  } else if (backward) {
+    if (D >= 64 && grid > 2048) return false;
+    if (D >= 64 && rows <= 640 && !(few || (grid <= 448 && D == 64))) limit = 0.96;
+  } else if (D == 128 && walk <= 512 && !few) {
+    limit = 0.95;
+  }
+  return split_share(p, heads) <= limit;
 }
 
 hipError_t launch_f32_fwd(int D, const void* q, const void* k, const void* v, void* o, float* lse,

@@ -31,7 +31,7 @@ hipError_t launch_bwd16_dkdv(int dtype, int D, const void* q, const void* k, con
 hipError_t launch_bwd16_dq(int dtype, int D, const void* q, const void* k, const void* v,
                            const void* dout, const float* lse, const float* delta, void* dq,
                            const AttnParams& p, hipStream_t st);
-bool f32_split_walk(const AttnParams& p, int heads, bool backward);
+bool f32_split_walk(const AttnParams& p, int D, int heads, bool backward);
 hipError_t launch_f32_fwd(int D, const void* q, const void* k, const void* v, void* o, float* lse,
                           const AttnParams& p, hipStream_t st);
 hipError_t launch_f32_dq(int D, const void* q, const void* k, const void* v, const void* dout,
@@ -237,6 +237,11 @@ const char* mi_attn_error_string(int status) {
 
 int mi_attn_check(const mi_attn_shape* s) { return validate(s); }
 
+int mi_attn_f32_split(const mi_attn_shape* s, int pass) {
+  if (validate(s) || s->dtype != MI_F32 || empty(s) || pass < 0 || pass > 2) return 0;
+  return mi::f32_split_walk(params(s), s->D, pass == 2 ? s->Hkv : s->H, pass > 0) ? 1 : 0;
+}
+
 int mi_attn_bwd_workspace(const mi_attn_shape* s, long long* floats) {
   if (!floats) return MI_ERR_NULL;
   const int st = validate(s);
@@ -270,7 +275,7 @@ int run_fwd(const void* q, const void* k, const void* v, const float* gate, void
   p.o_res = o_res;
   const hipError_t e =
       s->dtype != MI_F32 ? mi::launch_fwd16(s->dtype, s->D, q, k, v, o, lse, p, stream)
-      : mi::f32_split_walk(p, s->H, false) ? mi::launch_f32_fwd(s->D, q, k, v, o, lse, p, stream)
+      : mi::f32_split_walk(p, s->D, s->H, false) ? mi::launch_f32_fwd(s->D, q, k, v, o, lse, p, stream)
                                           : mi::launch_fwd(s->dtype, s->D, q, k, v, o, lse, p, stream);
   if (e != hipSuccess) return MI_ERR_LAUNCH;
   return status_of(mi::launch_sink_fwd(s->dtype, s->D, q, k, v, o, lse, p, stream));
@@ -351,7 +356,7 @@ int run_dkdv(const void* q, const void* k, const void* v, const void* dout, cons
   const hipError_t e =
       s->dtype != MI_F32
           ? mi::launch_bwd16_dkdv(s->dtype, s->D, q, k, v, dout, lse, delta, dk, dv, p, stream)
-      : mi::f32_split_walk(p, s->Hkv, true)
+      : mi::f32_split_walk(p, s->D, s->Hkv, true)
           ? mi::launch_f32_dkdv(s->D, q, k, v, dout, lse, delta, dk, dv, p, stream)
           : mi::launch_bwd_dkdv(s->dtype, s->D, q, k, v, dout, lse, delta, dk, dv, p, stream);
   if (e != hipSuccess) return MI_ERR_LAUNCH;
@@ -385,7 +390,7 @@ int run_dq(const void* q, const void* k, const void* v, const void* dout, const 
   const hipError_t e =
       s->dtype != MI_F32
           ? mi::launch_bwd16_dq(s->dtype, s->D, q, k, v, dout, lse, delta, dq, p, stream)
-      : mi::f32_split_walk(p, s->H, true)
+      : mi::f32_split_walk(p, s->D, s->H, true)
           ? mi::launch_f32_dq(s->D, q, k, v, dout, lse, delta, dq, p, stream)
           : mi::launch_bwd_dq(s->dtype, s->D, q, k, v, dout, lse, delta, dq, p, stream);
   if (e != hipSuccess) return MI_ERR_LAUNCH;
@@ -434,7 +439,7 @@ int run_bwd(const void* q, const void* k, const void* v, const float* gate, cons
   if (!q || !k || !v || !o || !dout || !lse || !delta || !dq || !dk || !dv) return MI_ERR_NULL;
   const mi::AttnParams p = params(s);
   const void* g = gate ? dout_attn : dout;
-  if (s->dtype != MI_F32 || (!gate && mi::f32_split_walk(p, s->H, true))) {
+  if (s->dtype != MI_F32 || (!gate && mi::f32_split_walk(p, s->D, s->H, true))) {
     // A dQ kernel that can computes the delta pass itself and runs first; dK/dV
     // (and the sink pass) then read the planes it wrote.
     if (!aligned16(o) || !aligned16(delta)) return MI_ERR_ALIGN;

@@ -1006,8 +1006,8 @@ def test_f32_split_walk_edges(D, T, mode):
 @pytest.mark.parametrize("B,T,D,window", [(64, 100, 64, 0), (64, 127, 32, 0), (32, 300, 64, 40),
                                           (24, 100, 128, 0)])
 def test_f32_full_chip_short_walks(B, T, D, window):
-    """Many heads with short walks: the 128-row float32 kernels (the launches that the
-    split walk leaves to them)."""
+    """Many heads with short walks: grids on both sides of where the split walk leaves
+    launches to the 128-row float32 kernels (F32_TILED below has all of theirs)."""
     H = 12
     q, k, v, do = _rand(B, T, H, H // 2, D, torch.float32, seed=T)
     scale = 1.0 / math.sqrt(D)
@@ -1134,3 +1134,44 @@ def test_gated_delta_inside_dq_has_the_bits_of_the_passes(dtype, D, mode, with_d
         outs.append([dq, dk, dv, dz, doa, ws[:2 * B * H * T]])
     for n, a, b in zip(("dQ", "dK", "dV", "dgate", "sigma dO", "planes"), *outs):
         assert torch.equal(a, b), n
+
+
+# float32 launches that stay on the 128-row kernels, by mi_attn_f32_split's passes (0
+# forward, 1 dQ, 2 dK/dV; tests/test_host.py checks the routes): (passes, mode, B, T, H, Hkv).
+F32_TILED = [((0, 1, 2), m, 86, t, 12, 6) for m, t in (("causal", 100), ("noncausal", 127),
+                                                       ("blocks", 100), ("window+sinks", 100),
+                                                       ("gated", 97))] \
+    + [((0, 1, 2), "noncausal", 21, 256, 12, 12), ((1, 2), "causal", 86, 300, 12, 6)]
+
+
+def f32_mode(mode):
+    """(causal, window, sinks, block) of a mode."""
+    return mode != "noncausal", *((40, 3) if "sinks" in mode else (0, 0)), 7 if mode == "blocks" else 0
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("case", F32_TILED, ids=lambda c: "%s_B%dT%dH%d_%d" % c[1:])
+def test_f32_128_row_kernels(case, D):
+    """The 128-row float32 kernels: every D and mask, a gate, GQA, one and several tiles
+    a walk; three batches of each against the oracle."""
+    _, mode, B, T, H, Hkv = case
+    causal, window, sinks, block = f32_mode(mode)
+    g = torch.Generator(device="cuda").manual_seed(T + D)
+    q, k, v, do = (torch.randn(B, T, h, D, device="cuda", generator=g) for h in (H, Hkv, Hkv, H))
+    z = torch.randn(B, T, H, device="cuda", generator=g) if mode == "gated" else None
+    scale = 1.0 / math.sqrt(D)
+    xs = [t.requires_grad_() for t in (q, k, v)]
+    o, lse = fc.attn(*xs, causal, window, scale, sinks=sinks, gate=z, block=block)
+    grads = torch.autograd.grad(o, xs, do)
+    for b in (0, B // 2, B - 1):
+        qb, kb, vb, db, zb = (None if t is None else t[b:b + 1].detach().cpu() for t in (q, k, v, do, z))
+        if z is None:
+            ow, lw = orc.forward(qb, kb, vb, scale, causal, window, sinks=sinks, block=block)
+            want = [ow, lw, *orc.backward(qb, kb, vb, ow, lw, db, scale, causal, window,
+                                          sinks=sinks, block=block)]
+        else:
+            ow, lw = orc.forward_gated(qb, kb, vb, zb, scale, causal, window, sinks)
+            want = [ow, lw, *orc.backward_gated(qb, kb, vb, zb, ow, lw, db, scale, causal, window,
+                                                sinks=sinks)[:3]]
+        got = [t[b:b + 1].detach().double().cpu().numpy() for t in (o, lse, *grads)]
+        _compare(got, want, torch.float32, f"f32 128 rows {mode} T{T} D{D} b{b}")

@@ -252,3 +252,41 @@ def test_backward_workspace_gqa_split():
     assert floats(B=1, S=32768, H=32, Hkv=1, D=128) == 2 * 32 * 32768
     # The reference's E17 shape (B8 T1024 H12/Hkv4 D32): 256 workgroups -> split.
     assert floats(B=8, S=1024, H=12, Hkv=4, D=32) == split(8, 1024, 12, 32, 2 * 8 * 12 * 1024)
+
+
+# ---------------------------------------------------------------------------
+# float32: which kernels a launch takes (mi_attn_f32_split)
+# ---------------------------------------------------------------------------
+def _f32_split(B, T, H, Hkv, D, mode="causal", window=0, dtype=None):
+    import ctypes
+    from tests.test_gpu_parity import f32_mode
+    causal, w, sinks, block = f32_mode(mode)
+    shp = _capi.shape(B, T, H, Hkv, D, causal, window or w, D ** -0.5,
+                      _capi.MI_F32 if dtype is None else dtype, sinks, block)
+    return tuple(_capi.load().mi_attn_f32_split(ctypes.byref(shp), i) for i in range(3))
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_f32_tests_run_the_kernels_they_name(D):
+    from tests.test_gpu_parity import F32_TILED
+    for passes, mode, B, T, H, Hkv in F32_TILED:
+        got = _f32_split(B, T, H, Hkv, D, mode)
+        assert all(got[i] == 0 for i in passes), (mode, B, T, got)
+    for T in (1, 31, 33, 127, 129, 161):                     # test_f32_split_walk_edges
+        for mode in ("causal", "noncausal", "blocks"):
+            assert _f32_split(2, T, 6, 2, D, mode) == (1, 1, 1)
+        assert _f32_split(2, T, 6, 2, D, window=33) == (1, 1, 1)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_f32_split_walk_limits(D):
+    """Few workgroups split; a chip that is full either way with walks of 100-256 rows does
+    not; other types and empty calls are none of it; huge shapes do not overflow."""
+    assert _f32_split(4, 256, 4, 4, D) == (1, 1, 1)
+    assert _f32_split(1, 4096, 8, 2, D) == (1, 1, 1)
+    assert _f32_split(42, 128, 12, 12, D, "noncausal") == (0, 0, 0)
+    assert _f32_split(63, 256, 12, 12, D, "noncausal") == (0, 0, 0)
+    assert _f32_split(2, 2048, 96, 96, D) == ((1, 0, 0) if D > 32 else (1, 1, 1))
+    assert _f32_split(4, 256, 4, 4, D, dtype=_capi.MI_BF16) == (0, 0, 0)
+    assert _f32_split(0, 256, 4, 4, D) == (0, 0, 0)
+    assert _f32_split(1, 1 << 24, 4, 4, D) == (0, 0, 0)
