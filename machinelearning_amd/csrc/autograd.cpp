@@ -9,7 +9,7 @@
 // small training step is bound by that host path: forward + backward of a small
 // attention call 118 -> 74 us, of a small prologue 122 -> 62 us (one box, medians;
 // torch's own `mul` takes 55 us forward + backward there). A call that a tracer
-// records keeps the Python nodes (flash_cuda._recorded).
+// records keeps the Python nodes (flash_cuda._python_node).
 #include <Python.h>
 
 #include <ATen/ATen.h>

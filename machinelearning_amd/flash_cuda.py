@@ -66,7 +66,7 @@ _DTYPE_CODE = {torch.float32: _capi.MI_F32, torch.float16: _capi.MI_F16,
                torch.bfloat16: _capi.MI_BF16}
 
 _lib = None
-_ext = None          # the C++ autograd nodes (csrc/autograd.cpp), imported with the library
+_ext = None          # the C++ autograd nodes (csrc/autograd.cpp); None: the Python ones run
 _load_error: str | None = None
 _load_attempted = False
 _mma_ok = False
@@ -130,11 +130,17 @@ def _load():
         return None
     try:
         lib = _capi.load()
-        from . import _mi_torch as ext
-    except (OSError, ImportError) as e:
-        _load_error = f"{type(e).__name__}: {e}"
+    except OSError as e:
+        _load_error = f"OSError: {e}"
         log.warning("libmi_attn.so did not load (%s)", _load_error)
         return None
+    try:
+        from . import _mi_torch as ext
+    except (OSError, ImportError) as e:
+        # Not built, or against another torch: the Python nodes launch the same kernels.
+        ext = None
+        log.warning("the C++ autograd nodes did not load (%s: %s); the Python ones run",
+                    type(e).__name__, e)
     _lib, _ext = lib, ext
     _mma_ok, _mma_error = True, None
     for dt in MMA_DTYPES:
@@ -344,8 +350,8 @@ class _AttnFn(torch.autograd.Function):
     The LSE tape [B,H,S] is saved for the backward, like the reference's
     ``_FlashAttnFn`` (``nanolab/flash_cuda.py:205-230``); its incoming
     gradient folds into Delta inside the library. ``_apply`` takes the same node
-    in C++ (``csrc/autograd.cpp``) wherever the call is plain eager; this
-    one is what a tracer can record.
+    in C++ (``csrc/autograd.cpp``) wherever the call is plain eager and that
+    loaded; this one is what a tracer can record.
     """
 
     @staticmethod
@@ -368,14 +374,16 @@ class _AttnFn(torch.autograd.Function):
         return dq, dk, dv, None, None, None, None, dgate, None
 
 
-def _recorded() -> bool:
-    """Whether a tracer records this call (``torch.jit.trace`` keeps a Python node as an
-    operator; Dynamo reads one): it then takes the Python autograd node."""
-    return torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
+def _python_node() -> bool:
+    """Whether this call takes the Python autograd node: a tracer records it
+    (``torch.jit.trace`` keeps a Python node as an operator; Dynamo reads one), or the C++
+    nodes did not load."""
+    return (torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
+            or _ext is None)
 
 
 def _apply(q, k, v, causal, window, sinks, scale, gate, block):
-    if _recorded():
+    if _python_node():
         return _AttnFn.apply(q, k, v, causal, window, sinks, scale, gate, block)
     return _ext.attn(q, k, v, gate, causal, window, sinks, scale, block,
                      _wants_residual(q, sinks, gate, window))

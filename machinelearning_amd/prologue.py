@@ -39,8 +39,8 @@ def _ptr(t):
 
 
 class _ProFn(torch.autograd.Function):
-    """The op's autograd node for a tracer (``flash_cuda._recorded``); eager calls take
-    the same node in C++ (``csrc/autograd.cpp``)."""
+    """The op's Python autograd node (``flash_cuda._python_node`` says for which calls);
+    eager ones take the same node in C++ (``csrc/autograd.cpp``)."""
 
     @staticmethod
     def forward(ctx, x, weight, cos, sin, eps, out_dtype):
@@ -120,6 +120,6 @@ def qk_norm_rope(x: torch.Tensor, weight: torch.Tensor | None, cos: torch.Tensor
     if x.numel() == 0:
         out = x.to(out_dtype)
         return out if w is None else out + 0.0 * w.sum().to(out_dtype)
-    if _fc._recorded():
+    if _fc._python_node():
         return _ProFn.apply(x, w, c, s, float(eps), out_dtype)
     return _fc._ext.prologue(x, w, c, s, float(eps), _CODE[out_dtype])

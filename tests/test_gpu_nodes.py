@@ -136,3 +136,29 @@ def test_transforms_are_refused_and_traces_run():
     traced = torch.jit.trace(lambda a, b, c: fc.attn(a, b, c)[0], (q, k, v))
     q2, k2, v2, _ = _qkv(B=1, seed=3)
     assert torch.equal(traced(q2, k2, v2), fc.attn(q2, k2, v2)[0])
+
+
+def test_without_the_cpp_nodes_everything_runs_on_the_python_ones(monkeypatch, caplog):
+    """A missing or foreign _mi_torch.so costs host time, not the library: attention,
+    prologue and decode run, with the same bits."""
+    import sys
+    import machinelearning_amd as pkg
+    from machinelearning_amd.decode import attn_cached
+
+    def step():
+        q, k, v, do = _qkv()
+        q.requires_grad_()
+        o, lse = fc.attn(q, k, v)
+        dq, = torch.autograd.grad(o, q, do)
+        y = pro.qk_norm_rope(do, torch.ones(64, device="cuda"), None, None)
+        with torch.no_grad():
+            return [o.detach(), lse.detach(), dq, y, attn_cached(q, k, v, {}, False, True)]
+    want = step()
+    monkeypatch.delattr(pkg, "_mi_torch")
+    monkeypatch.setitem(sys.modules, "machinelearning_amd._mi_torch", None)
+    for name, value in (("_lib", None), ("_ext", None), ("_load_attempted", False)):
+        monkeypatch.setattr(fc, name, value)
+    with caplog.at_level("WARNING"):
+        assert fc.is_available(), fc.unavailable_reason()
+    assert fc._ext is None and "autograd nodes did not load" in caplog.text
+    assert all(torch.equal(a, b) for a, b in zip(step(), want))
