@@ -355,8 +355,9 @@ MI_API int mi_attn_decode(const void* q, const void* k_new, const void* v_new,
  * rows [cache | new] those at positions < sinks or >= start + T - (window -
  * sinks - 1) stay, in their order. mi_attn_cache_plan writes the kept rows'
  * indices to `rows` (int32, cached + T), their positions to `positions`
- * (int64, cached + T) and how many there are to `count` (int32; device memory
- * or pinned host memory, readable once the call's work on `stream` is done). */
+ * (int64, cached + T; both may be NULL if there are no rows) and how many there
+ * are to `count` (int32; device memory or pinned host memory, readable once the
+ * call's work on `stream` is done). */
 MI_API int mi_attn_cache_plan(const long long* cache_pos, const mi_decode_shape* s, int* rows,
                               long long* positions, int* count, hipStream_t stream);
 

@@ -719,7 +719,7 @@ int mi_attn_cache_plan(const long long* cache_pos, const mi_decode_shape* s, int
   const int st = validate_dec(s);
   if (st) return st;
   if (s->window <= 0) return MI_ERR_WINDOW;
-  if (!rows || !positions || !count) return MI_ERR_NULL;
+  if (!count || ((long long)s->cached + s->T > 0 && (!rows || !positions))) return MI_ERR_NULL;
   const long long end = (long long)s->start + s->T;
   return status_of(mi::launch_cache_plan(cache_pos, s->cached, s->T, s->start,
                                          end - (s->window - s->sinks - 1), s->sinks, rows,

@@ -514,11 +514,12 @@ def test_decode_random_sweep(case):
 @pytest.mark.parametrize("Lc,T,window,sinks,evicted", [
     (0, 1, 4, 1, False), (0, 9, 1, 0, False), (3, 2, 64, 4, False), (254, 1, 300, 4, False),
     (62, 1, 64, 4, True), (255, 2, 256, 0, True), (255, 1, 2, 1, True), (513, 40, 300, 17, True),
-    (31, 3, 1, 0, True)])
+    (31, 3, 1, 0, True), (0, 0, 4, 1, False), (5, 0, 64, 4, False), (300, 0, 64, 4, True)])
 def test_window_commit_equals_boolean_indexing(dtype, Lc, T, window, sinks, evicted):
     """The committed window cache == the live rows of cat([cache, block]) by boolean
     indexing (mixers.py:437-448), whole values: row counts around the plan's 256-row
-    chunks, nothing left (window 1), positions in no order, a strided cache view."""
+    chunks, nothing left (window 1), positions in no order, a strided cache view, an
+    empty block (also on an empty cache)."""
     from machinelearning_amd.decode import attn_cached
     g = torch.Generator(device="cuda").manual_seed(Lc * 7 + T)
     B, H, Hkv, D = 2, 4, 2, 32
