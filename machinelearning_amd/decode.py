@@ -145,10 +145,15 @@ class _WindowCommit:
     and its count written to pinned memory: the wait is for the plan only, under
     the step. Without ``pos`` (nothing evicted yet) the count follows from the
     lengths, and nothing is waited for.
+
+    torch's pinned allocator does not know that a kernel writes the count, so it
+    must not get that memory back before the plan has run: an object dropped
+    unread (the step failed) waits for the device.
     """
 
     def __init__(self, lib, shp, cpos, Lc, T, start, window, sinks, dev, stream):
         n = Lc + T
+        self.known, self.dev = 0, dev
         self.rows = torch.empty(n + 1, dtype=torch.int32, device=dev)
         self.pos = torch.empty(n, dtype=torch.int64, device=dev)
         if cpos is None:
@@ -156,18 +161,21 @@ class _WindowCommit:
             self.known = lead + end - max(lead, end - (window - sinks - 1), 0)
             self.count, self.done = self.rows[n:], None
         else:
-            self.known = None
             self.count = torch.empty(1, dtype=torch.int32, pin_memory=True)
             self.done = torch.cuda.Event()
+            self.known = None
         _capi.check(lib.mi_attn_cache_plan(None if cpos is None else cpos.data_ptr(),
                                            ctypes.byref(shp), self.rows.data_ptr(),
                                            self.pos.data_ptr(), self.count.data_ptr(), stream))
         if self.done is not None:
             self.done.record()
 
+    def __del__(self):
+        if self.known is None:
+            torch.cuda.synchronize(self.dev)
+
     def wait(self) -> int:
-        """Rows that stay. (Also called when the step fails: the pinned count must
-        outlive the plan that writes it.)"""
+        """Rows that stay."""
         if self.known is None:
             self.done.synchronize()
             self.known = int(self.count[0])
@@ -293,20 +301,17 @@ def attn_cached(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache: dict, 
 
     with _fc._on_device(q):
         stream = _fc._stream(q)
+        ws = _workspace(dev, stream, nws) if nws > 0 else None
         kept = (_WindowCommit(lib, shp, cpos, Lc, T, start, window, sinks, dev, stream)
                 if commit and window else None)
-        ws = _workspace(dev, stream, nws) if nws > 0 else None
         st = lib.mi_attn_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), ptr(ck), ptr(cv),
                                 ptr(cpos), ptr(g), out.data_ptr(), ptr(lse), ptr(ws),
                                 ctypes.byref(shp), stream)
+        _capi.check(st)
         if kept is not None:
-            if st:
-                kept.wait()
-            else:
-                # Keep the sinks plus the tail the next block can still reach
-                # (mixers.py:437-448).
-                kept.store(lib, shp, cache, k, v, ck, cv, stream, start + T)
-    _capi.check(st)
+            # Keep the sinks plus the tail the next block can still reach
+            # (mixers.py:437-448).
+            kept.store(lib, shp, cache, k, v, ck, cv, stream, start + T)
 
     if commit and not window:
         kt, vt = k.transpose(1, 2), v.transpose(1, 2)          # (B, Hkv, T, D) views

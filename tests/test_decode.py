@@ -638,3 +638,39 @@ def test_decode_two_to_four_rows_hold_p_in_fp32(dtype, keys):
     tol = _parity.half_ulp(ref.cpu().numpy(), dtype) + 1e-6 * mag.cpu().numpy()
     print(f"decode P fp32 {dtype} {keys}: worst err/tol {(err / tol).max():.3f}", flush=True)
     assert (err <= tol).all(), (int((err > tol).sum()), err.size)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fails", ["workspace", "step"])
+def test_failed_windowed_step_waits_before_its_pinned_count_is_freed(monkeypatch, fails):
+    """A committed step that fails after (or before) its plan is launched: the plan's kernel
+    writes a pinned count, so the device is waited for before that memory goes back; the
+    cache stays as it was, and the step then succeeds on it."""
+    import gc
+    from machinelearning_amd import _capi
+    from machinelearning_amd import decode
+    lib = _capi.load()
+    log = []
+    plan, sync = lib.mi_attn_cache_plan, torch.cuda.synchronize
+    monkeypatch.setattr(lib, "mi_attn_cache_plan", lambda *a: (log.append("plan"), plan(*a))[1])
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: (log.append("wait"), sync(*a))[1])
+    B, T, H, D, Lc = 1, 1, 4, 64, 4000          # long enough to split: a workspace
+    q, k, v = (torch.randn(B, T, H, D, device="cuda") for _ in range(3))
+    start = {"k": torch.randn(B, H, Lc, D, device="cuda"), "v": torch.randn(B, H, Lc, D, device="cuda"),
+             "pos": torch.arange(10, Lc + 10, device="cuda"), "end": Lc + 10}
+    cache = dict(start)
+    with torch.no_grad(), monkeypatch.context() as m:
+        if fails == "workspace":
+            def no_memory(*a):
+                raise MemoryError("no workspace")
+            m.setattr(decode, "_workspace", no_memory)
+        else:
+            m.setattr(lib, "mi_attn_decode", lambda *a: 1)
+        with pytest.raises((MemoryError, RuntimeError)):
+            decode.attn_cached(q, k, v, cache, True, True, window=4096, sinks=4)
+    gc.collect()
+    assert log == ([] if fails == "workspace" else ["plan", "wait"])
+    assert cache == start
+    with torch.no_grad():
+        decode.attn_cached(q, k, v, cache, True, True, window=4096, sinks=4)
+    assert log[-1] == "plan" and cache["end"] == Lc + 11 and cache["k"].shape[2] == Lc + 1
