@@ -20,6 +20,7 @@
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/pybind.h>
 
 #include "../../include/mi_attn.h"
 
@@ -243,8 +244,13 @@ PyObject* py_attn(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (PyErr_Occurred()) throw python_error();
   const bool keep = res && at::GradMode::is_enabled() &&
                     (q.requires_grad() || k.requires_grad() || v.requires_grad());
-  variable_list out =
-      Attn::apply(q, k, v, maybe(gate), causal, window, sinks, scale, block, keep);
+  variable_list out;
+  {
+    // As torch's own operators: an allocation may block, or want the GIL for a
+    // callback under the allocator's lock.
+    pybind11::gil_scoped_release no_gil;
+    out = Attn::apply(q, k, v, maybe(gate), causal, window, sinks, scale, block, keep);
+  }
   PyObject* o = THPVariable_Wrap(std::move(out[0]));
   if (!o) throw python_error();
   PyObject* lse = THPVariable_Wrap(std::move(out[1]));
@@ -274,7 +280,12 @@ PyObject* py_prologue(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const double eps = PyFloat_AsDouble(args[4]);
   const int64_t code = PyLong_AsLongLong(args[5]);
   if (PyErr_Occurred()) throw python_error();
-  return THPVariable_Wrap(Prologue::apply(x, maybe(w), maybe(c), maybe(s), eps, code));
+  Tensor out;
+  {
+    pybind11::gil_scoped_release no_gil;
+    out = Prologue::apply(x, maybe(w), maybe(c), maybe(s), eps, code);
+  }
+  return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
 

@@ -162,3 +162,41 @@ def test_without_the_cpp_nodes_everything_runs_on_the_python_ones(monkeypatch, c
         assert fc.is_available(), fc.unavailable_reason()
     assert fc._ext is None and "autograd nodes did not load" in caplog.text
     assert all(torch.equal(a, b) for a, b in zip(step(), want))
+
+
+@pytest.mark.parametrize("node", ["attn", "prologue"])
+def test_the_nodes_release_the_gil(node):
+    """Other Python threads run while a node allocates and launches. The switch interval is
+    set so long that the second thread, which wakes from a sleep, gets the GIL only
+    where the call gives it up."""
+    import sys
+    import threading
+    import time
+    q, k, v, do = _qkv()
+    call = {"attn": lambda: fc._ext.attn(q, k, v, None, True, 0, 0, 0.125, 0, False),
+            "prologue": lambda: fc._ext.prologue(do, None, None, None, 1e-6, 2)}[node]
+    call()
+    turns, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            turns[0] += 1
+            time.sleep(1e-4)
+    thread = threading.Thread(target=other)
+    interval = sys.getswitchinterval()
+    try:
+        sys.setswitchinterval(1000.0)
+        thread.start()
+        time.sleep(0.01)
+        before = turns[0]
+        kept = []                                # freeing a tensor may give the GIL up too
+        for _ in range(8000):
+            kept.append(call())
+            if turns[0] > before:
+                break
+        gained = turns[0] - before
+    finally:
+        sys.setswitchinterval(interval)
+        stop.set()
+        thread.join()
+    assert gained > 0
