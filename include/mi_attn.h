@@ -216,6 +216,15 @@ MI_API int mi_attn_bwd_gated(const void* q, const void* k, const void* v, const 
                              void* dk, void* dv, float* dgate, const mi_attn_shape* s,
                              hipStream_t stream);
 
+/* The gated backward without an LSE gradient in bfloat16 (others: MI_ERR_DTYPE) with
+ * one rounding less: sigma = sigmoid(gate) enters dS = sigma P (dout V^T - Delta /
+ * sigma) and dV = (sigma P)^T dout through P. `dout_attn` receives dout, divided by
+ * 2^64 in rows of logits under -60 (where sigma P alone would be flushed). */
+MI_API int mi_attn_bwd_gated_direct(const void* q, const void* k, const void* v, const float* gate,
+                                    const void* o, const void* dout, const float* lse,
+                                    float* delta, void* dout_attn, void* dq, void* dk, void* dv,
+                                    float* dgate, const mi_attn_shape* s, hipStream_t stream);
+
 /* Stage 1 of the gated backward: mi_attn_bwd_delta plus dout_attn and dgate
  * (as above). Stages 2 and 3 are then mi_attn_bwd_dkdv / mi_attn_bwd_dq with
  * dout_attn in place of dout. */

@@ -92,6 +92,7 @@ SIGNATURES = {
     "mi_attn_bwd_res": (ctypes.c_int, [_P] * 12 + [_SHAPE, _P]),
     "mi_attn_fwd_gated": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _SHAPE, _P]),
     "mi_attn_bwd_gated": (ctypes.c_int, [_P] * 14 + [_SHAPE, _P]),
+    "mi_attn_bwd_gated_direct": (ctypes.c_int, [_P] * 13 + [_SHAPE, _P]),
     "mi_attn_bwd_delta_gated": (ctypes.c_int, [_P] * 8 + [_SHAPE, _P]),
     "mi_attn_bwd_dkdv": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _SHAPE, _P]),
     "mi_attn_bwd_dq": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _SHAPE, _P]),

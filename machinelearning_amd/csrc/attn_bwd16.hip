@@ -98,18 +98,23 @@ __host__ __device__ inline long long split_pitch(int S) { return (S + 127LL) / 1
 // query row is owned by exactly one lane pair, so every plane entry is written
 // once.
 //
-// GATE (with FD): O and dO are those of the gated output y = sigma O. The kernel
-// then also does the rest of the delta pass (attn_bwd_delta_kernel): dS = P
-// (sigma dO V^T - Delta) takes the rows sigma * dO, rounded to T, which it
-// writes to p.doe for dK/dV, and the gate's gradient is (1 - sigma) rowsum(dO * y).
-// Sums and roundings are those of the delta pass, so the results are its bits.
-// (sigma stays with dO: sigma P would leave float16's range at logits of -4 and
-// bfloat16's near -80, where sigma * dO is still in it.) Backward with the delta
-// launch -> without, us: board shape bf16 135.5 -> 127.0 (ungated 121.4), f16
-// 136.5 -> 130.0; f16 B5 S777 H9/3 D64, blocks of 32: 51.0 -> 47.3; bf16 B2
-// S4096 H16 D128: 547 -> 537.
+// With FD and a gate, O and dO are those of the gated output y = sigma O; the kernel
+// then also writes the rows of p.doe, which dK/dV reads in place of dO, and the
+// gate's gradient, (1 - sigma) rowsum(dO * y). dS = P (sigma dO V^T - Delta).
+// kGateRows: sigma * dO, rounded to T. Sums and roundings are those of the delta
+//   pass (attn_bwd_delta_kernel), so the results are its bits.
+// kGateFold (bfloat16): sigma in P instead, one rounding less: dS = (sigma P)(dO
+//   V^T - Delta / sigma), dV = (sigma P)^T dO, with the planes Delta / sigma and
+//   (ln sigma - LSE) / scale. Rows of logits under -60, whose sigma P would be
+//   flushed (near -80 all of it), take dO / 2^64, exact, and 2^64 sigma. Not for
+//   float16, where sigma P is subnormal from logits of -4 on. Relative error of
+//   the gradients, B16 S1024 H12 D64: 2.5e-3, 3.1e-3 with kGateRows.
+// Backward with the delta launch -> without, us: board shape bf16 135.5 -> 127.0
+// (ungated 121.4), f16 136.5 -> 130.0; f16 B5 S777 H9/3 D64, blocks of 32: 51.0 ->
+// 47.3; bf16 B2 S4096 H16 D128: 547 -> 537.
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool BLK, bool FD, bool GATE = false>
+enum { kGateNone = 0, kGateRows = 1, kGateFold = 2 };
+template <typename T, int D, bool BLK, bool FD, int GATE = kGateNone>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2, 8)))
 attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
                      const T* __restrict__ dO, const float* __restrict__ LSE,
@@ -149,11 +154,14 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
   // This row's LSE (and LSE gradient), loaded up front: with O by DMA the
   // delta is finished only after the ring's first wait.
   const long long ridx = ((long long)b * p.H + h) * p.S + qi;
-  float Lrow = 0.f, dlrow = 0.f, sg = 1.f;
+  float Lrow = 0.f, dlrow = 0.f, sg = 1.f, zrow = 0.f;
   if (FD && qi < p.S) {
     Lrow = LSE[ridx];
     if (p.dlse) dlrow = p.dlse[ridx];
-    if constexpr (GATE) sg = gate_sigmoid(p, b, qi, h);
+    if constexpr (GATE != kGateNone) {
+      zrow = p.gate[((long long)b * p.S + qi) * p.H + h];
+      sg = 1.f / (1.f + __expf(-zrow));
+    }
   }
   // Fused delta, given this lane's partial dot product of dO and O (head dims
   // {16 ds + 8 g + e} of row qi; the lane 32 away holds the other half).
@@ -161,14 +169,23 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
     Dq = halves_sum(part);
     if (qi < p.S) {
       const long long idx = ridx;
-      const float L = Lrow;
-      if constexpr (GATE) {
+      float L = Lrow;
+      if constexpr (GATE != kGateNone) {
+        float mul = sg;   // of the row of dO
         if (g == 0) p.dgate[((long long)b * p.S + qi) * p.H + h] = (1.f - sg) * Dq;
+        if constexpr (GATE == kGateFold) {
+          // e = 1 / sigma, or that over 2^64 (logits from -130 on are 0 either way).
+          const bool low = zrow < -60.f;
+          const float e = low ? __expf(fminf(-zrow, 130.f) - 44.36141956f) : 1.f + __expf(-zrow);
+          mul = low ? 0x1p-64f : 1.f;
+          Dq *= e;
+          L += logf(e);
+        }
         T* doe = reinterpret_cast<T*>(p.doe) + ((long long)b * p.S + qi) * p.q_rs + (long long)h * D;
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) dof[ds][e] = (T)((float)dof[ds][e] * sg);
+          for (int e = 0; e < 8; ++e) dof[ds][e] = (T)((float)dof[ds][e] * mul);
           *reinterpret_cast<frag*>(doe + ds * 16 + g * 8) = dof[ds];
         }
       }
@@ -180,18 +197,19 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
       }
     }
   };
-  // This lane's partial of rowsum(dO * O), chunk ds of O at a time. GATE: each
+  // This lane's partial of rowsum(dO * O), chunk ds of O at a time. kGateRows: each
   // chunk summed by itself, the chunks in the delta pass's order.
-  float part = 0.f, chunk[GATE ? DS : 1];
+  constexpr bool BY_CHUNK = GATE == kGateRows;
+  float part = 0.f, chunk[BY_CHUNK ? DS : 1];
   auto add_chunk = [&](int ds, const frag& of) __attribute__((always_inline)) {
-    float x = GATE ? 0.f : part;
+    float x = BY_CHUNK ? 0.f : part;
 #pragma unroll
     for (int e = 0; e < 8; ++e) x = fmaf((float)of[e], (float)dof[ds][e], x);
-    if constexpr (GATE) chunk[ds] = x;
+    if constexpr (BY_CHUNK) chunk[ds] = x;
     else part = x;
   };
   auto row_part = [&]() __attribute__((always_inline)) {
-    if constexpr (GATE) {
+    if constexpr (BY_CHUNK) {
 #pragma unroll
       for (int x = DS / 2; x >= 1; x >>= 1)
 #pragma unroll
@@ -224,7 +242,7 @@ attn_bwd16_dq_kernel(const T* __restrict__ Q, const T* __restrict__ K, const T* 
         for (int j = 0; j < C::LPW; ++j)
           dma16_buf(ro, ooff[j], m0o + (unsigned)(half * C::TILE + 4096 * j));
       }
-    } else if (!GATE && p.o_res) {
+    } else if (GATE == kGateNone && p.o_res) {
       // O as stored plus its rounding residual: Delta from O to ~16 bits
       // (with O alone, its 8-bit rounding enters every dS of the row).
       const T* Rb = reinterpret_cast<const T*>(p.o_res) + hoff;
@@ -910,7 +928,7 @@ static hipError_t launch_dq16_t(const void* q, const void* k, const void* v, con
   const long long nblocks = (long long)p.nblk * p.B * p.H;
   p.wi_blocks_fastest = !p.causal;
   p.div_wi = p.wi_blocks_fastest ? work_item_div_blocks(p.nblk) : work_item_div((long long)p.B * p.H);
-  // Variants: block-causal (BLK) x delta fused in (FD, when p.o is set), gated or not.
+  // Variants: block-causal (BLK) x delta fused in (FD, when p.o is set), and how a gate enters.
   const auto go = [&](auto blk_c, auto fd_c, auto gate_c) {
     hipLaunchKernelGGL((attn_bwd16_dq_kernel<T, D, decltype(blk_c)::value, decltype(fd_c)::value,
                                              decltype(gate_c)::value>),
@@ -920,9 +938,12 @@ static hipError_t launch_dq16_t(const void* q, const void* k, const void* v, con
   using yes = std::true_type;
   using no = std::false_type;
   const auto by_fd = [&](auto blk_c) {
-    if (p.o && p.gate) go(blk_c, yes{}, yes{});
-    else if (p.o) go(blk_c, yes{}, no{});
-    else go(blk_c, no{}, no{});
+    if constexpr (std::is_same_v<T, __bf16>) {
+      if (p.o && p.gate && p.gate_fold) return go(blk_c, yes{}, ic<kGateFold>{});
+    }
+    if (p.o && p.gate) go(blk_c, yes{}, ic<kGateRows>{});
+    else if (p.o) go(blk_c, yes{}, ic<kGateNone>{});
+    else go(blk_c, no{}, ic<kGateNone>{});
   };
   if (p.block > 1) by_fd(yes{});
   else by_fd(no{});

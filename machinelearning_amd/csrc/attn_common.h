@@ -79,7 +79,8 @@ struct AttnParams {
   long long kv_rs;    // row stride of k/v/dk/dv in elements (Hkv * D)
   const float* gate;  // per-(b, i, h) output gate logits [B, S, H] (nullptr: no gate)
   float* dgate;       // fused delta pass of a gated backward: the logits' gradient
-  void* doe;          //   and sigmoid(gate) * dO, both written by the dQ kernel
+  void* doe;          //   and the rows dK/dV reads for dO, both written by the dQ kernel
+  int gate_fold;      //   sigmoid(gate) enters through P (bfloat16), not through doe
   // Backward with the delta pass fused into the 16-bit dQ kernel: O, the LSE
   // gradient (or nullptr) and the workspace whose two planes it fills
   // (o == nullptr: the planes were written by the delta kernel).

@@ -141,11 +141,16 @@ struct Attn : torch::autograd::Function<Attn> {
         check(mi_attn_bwd(ptr(q), ptr(k), ptr(v), ptr(o), ptr(dy), floats(lse), floats(dl),
                           floats(ws), ptr(dq), ptr(dk), ptr(dv), &s, st));
       } else {
-        const Tensor dy_attn = at::empty_like(dy);   // sigmoid(gate) * dy, the kernels' input
+        const Tensor dy_attn = at::empty_like(dy);   // the gradient of O as dK/dV reads it
         dz = at::empty_like(gate);
-        check(mi_attn_bwd_gated(ptr(q), ptr(k), ptr(v), floats(gate), ptr(o), ptr(dy), floats(lse),
-                                floats(dl), floats(ws), ptr(dy_attn), ptr(dq), ptr(dk), ptr(dv),
-                                floats(dz), &s, st));
+        if (!dl.defined() && s.dtype == MI_BF16)
+          check(mi_attn_bwd_gated_direct(ptr(q), ptr(k), ptr(v), floats(gate), ptr(o), ptr(dy),
+                                         floats(lse), floats(ws), ptr(dy_attn), ptr(dq), ptr(dk),
+                                         ptr(dv), floats(dz), &s, st));
+        else
+          check(mi_attn_bwd_gated(ptr(q), ptr(k), ptr(v), floats(gate), ptr(o), ptr(dy), floats(lse),
+                                  floats(dl), floats(ws), ptr(dy_attn), ptr(dq), ptr(dk), ptr(dv),
+                                  floats(dz), &s, st));
       }
       out = {dq, dk, dv, dz};
     }

@@ -166,6 +166,7 @@ mi::AttnParams params(const mi_attn_shape* s) {
   p.gate = nullptr;
   p.dgate = nullptr;
   p.doe = nullptr;
+  p.gate_fold = 0;
   p.o = nullptr;
   p.dlse = nullptr;
   p.ws_out = nullptr;
@@ -372,7 +373,7 @@ int run_dq(const void* q, const void* k, const void* v, const void* dout, const 
            const float* delta, void* dq, const mi_attn_shape* s, hipStream_t stream,
            SinkPass sp, const void* o = nullptr, const float* dlse = nullptr,
            const void* o_res = nullptr, const float* gate = nullptr, void* doe = nullptr,
-           float* dgate = nullptr) {
+           float* dgate = nullptr, bool gate_fold = false) {
   if (!q || !k || !v || !dout || !lse || !delta || !dq) return MI_ERR_NULL;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(dout) || !aligned16(dq) ||
       (o && !aligned16(o)) || (doe && !aligned16(doe)))
@@ -385,6 +386,7 @@ int run_dq(const void* q, const void* k, const void* v, const void* dout, const 
     p.o_res = const_cast<void*>(o_res);
     p.gate = gate;
     p.doe = doe;
+    p.gate_fold = gate_fold;
     p.dgate = dgate;
   }
   const hipError_t e =
@@ -554,6 +556,24 @@ int mi_attn_bwd_gated(const void* q, const void* k, const void* v, const float* 
   if (!gate || !dout_attn || !dgate) return MI_ERR_NULL;
   return run_bwd(q, k, v, gate, o, dout, lse, dlse, delta, dout_attn, dq, dk, dv, dgate, s,
                  stream);
+}
+
+int mi_attn_bwd_gated_direct(const void* q, const void* k, const void* v, const float* gate,
+                             const void* o, const void* dout, const float* lse, float* delta,
+                             void* dout_attn, void* dq, void* dk, void* dv, float* dgate,
+                             const mi_attn_shape* s, hipStream_t stream) {
+  const int st = validate(s);
+  if (st) return st;
+  if (s->dtype != MI_BF16) return MI_ERR_DTYPE;
+  if (empty(s)) return MI_OK;
+  if (!q || !k || !v || !gate || !o || !dout || !lse || !delta || !dout_attn || !dq || !dk || !dv ||
+      !dgate)
+    return MI_ERR_NULL;
+  if (!aligned16(o) || !aligned16(delta)) return MI_ERR_ALIGN;
+  const int r = run_dq(q, k, v, dout, lse, delta, dq, s, stream, SinkPass::kNone, o, nullptr, nullptr,
+                       gate, dout_attn, dgate, true);
+  if (r) return r;
+  return run_dkdv(q, k, v, dout_attn, lse, delta, dk, dv, s, stream, SinkPass::kNone);
 }
 
 namespace {

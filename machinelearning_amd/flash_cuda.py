@@ -331,14 +331,19 @@ def _bwd(do, dlse, q, k, v, o, lse, causal, window, sinks, scale, gate=None, blo
                                  None if dlse is None else dlse.data_ptr(), delta.data_ptr(),
                                  dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), sp, _stream(q))
         else:
-            do_attn = torch.empty_like(do)          # sigmoid(gate) * do, the kernels' input
+            do_attn = torch.empty_like(do)          # the gradient of O as dK/dV reads it
             dgate = torch.empty_like(gate)
-            st = lib.mi_attn_bwd_gated(q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                       gate.data_ptr(), o.data_ptr(), do.data_ptr(),
-                                       lse.data_ptr(), None if dlse is None else dlse.data_ptr(),
-                                       delta.data_ptr(), do_attn.data_ptr(), dq.data_ptr(),
-                                       dk.data_ptr(), dv.data_ptr(), dgate.data_ptr(), sp,
-                                       _stream(q))
+            if dlse is None and q.dtype == torch.bfloat16:
+                st = lib.mi_attn_bwd_gated_direct(
+                    q.data_ptr(), k.data_ptr(), v.data_ptr(), gate.data_ptr(), o.data_ptr(),
+                    do.data_ptr(), lse.data_ptr(), delta.data_ptr(), do_attn.data_ptr(),
+                    dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dgate.data_ptr(), sp, _stream(q))
+            else:
+                st = lib.mi_attn_bwd_gated(
+                    q.data_ptr(), k.data_ptr(), v.data_ptr(), gate.data_ptr(), o.data_ptr(),
+                    do.data_ptr(), lse.data_ptr(), None if dlse is None else dlse.data_ptr(),
+                    delta.data_ptr(), do_attn.data_ptr(), dq.data_ptr(), dk.data_ptr(),
+                    dv.data_ptr(), dgate.data_ptr(), sp, _stream(q))
     if st:
         _capi.check(st)
     return dq, dk, dv, dgate
