@@ -1,5 +1,5 @@
-// float32 attention for grids that leave the chip idle (gfx950): forward, dQ
-// (with the delta pass) and dK/dV whose workgroups split the walk.
+// float32 attention for grids that leave the chip idle, and for long walks (gfx950):
+// forward, dQ (with the delta pass) and dK/dV whose workgroups split the walk.
 //
 // v_mfma_f32_32x32x2f32 takes 64 cycles for 4 KFLOP, so a float32 wave is
 // bound by its serial chain of MFMAs: 128 per 32 x 64 tile forward, 256 in
