@@ -115,7 +115,8 @@ _lib = None
 # load, hipGetSymbolAddress, a launch that waits for queue space) and that are not on
 # the per-step autograd path: called through ctypes.CDLL, which releases the GIL.
 RELEASE_GIL = frozenset({"mi_attn_bwd_noalloc", "mi_attn_decode", "mi_attn_decode_workspace",
-                         "mi_mfma_probe", "mi_mfma_probe_k"})
+                         "mi_attn_cache_plan", "mi_attn_cache_gather", "mi_mfma_probe",
+                         "mi_mfma_probe_k"})
 
 
 class _Lib:

@@ -46,6 +46,7 @@ def test_gil_binding_per_entry_point():
         keeps = bool(getattr(lib, name)._flags_ & ctypes._FUNCFLAG_PYTHONAPI)
         assert keeps == (name not in _capi.RELEASE_GIL), name
     assert {"mi_attn_bwd_noalloc", "mi_attn_decode", "mi_mfma_probe"} <= _capi.RELEASE_GIL
+    assert {"mi_attn_cache_plan", "mi_attn_cache_gather"} <= _capi.RELEASE_GIL
     assert "mi_attn_fwd" not in _capi.RELEASE_GIL and "mi_attn_bwd" not in _capi.RELEASE_GIL
 
 
