@@ -486,22 +486,22 @@ static double split_share(const AttnParams& p, int heads) {
 // two waves per SIMD (and 4 / 15 spilled registers in dQ / dK/dV at D = 64): little on a
 // long walk, 10-25% on one of 100-250 rows of a chip that is full either way. The
 // limits are measured over 2100 shapes, each pass and D: none taken is over 5%
-// slower, three over 2.5%. 128-row kernels -> these, fwd / bwd us:
-//   causal   D64  grid 32    S256    28.7 -> 8.7     95.8 -> 28.4
-//            D64  grid 768   S1024    158 -> 126      507 -> 470
-//            D64  grid 504   S256    (causal bwd limit)   137 <- 151
-//            D128 grid 288   S1024    182 -> 119      606 -> 416
-//            D128 grid 1488  S256     271 <- 276      984 <- 1017
-//            D128 grid 3072  S2048   2357 -> 2228    7995 <- 8691
-//            D32  grid 768   S1024   86.8 -> 64.6     291 -> 237
-//   full     D64  grid 960   S1024    324 -> 277     1066 -> 976
-//            D64  grid 3000  S128     164 <- 189      609 <- (grid)
-//            D64  grid 1488  S256     142 -> 140      488 <- 557
-//            D128 grid 264   S256     109 -> 79       370 -> 266
-//            D128 grid 252   S128    36.5 <- 45.1     129 <- 143
-//            D32  grid 1488  S256    (fwd limit)      239 <- 265
-//   window   D64  grid 2048  256, S4096  254 -> 215   843 <- 861
-//            D128 grid 288   64, S3000  (0.52 of the time)
+// slower, three over 2.5%. 128-row kernels | these, fwd and bwd us, * the one taken:
+//   causal  D64  grid 32    S256     28.7 |   8.7*    95.8 |  28.4*
+//           D64  grid 768   S1024     158 |   126*     507 |   470*
+//           D32  grid 768   S1024    86.8 |  64.6*     291 |   237*
+//           D64  grid 504   S256                       137*|   151
+//           D128 grid 288   S1024     182 |   119*     606 |   416*
+//           D128 grid 1488  S256      271*|   276      984*|  1017
+//           D128 grid 3072  S2048    2357 |  2228*    7995*|  8691
+//   full    D64  grid 960   S1024     324 |   277*    1066 |   976*
+//           D64  grid 1488  S256      142*|   140      488*|   557
+//           D32  grid 1488  S256                       239*|   265
+//           D64  grid 3000  S128      164*|   189
+//           D128 grid 264   S256      109 |    79*     370 |   266*
+//           D128 grid 252   S128     36.5*|  45.1      129*|   143
+//   window  D64  grid 2048  256 of 4096 254 | 215*     843*|   861
+//           D128 grid 192   64 of 2048 45.5 | 28.1*    158 |  99.8*
 // Offsets inside a head and the row vectors are 32-bit here (S <= 2 GiB of rows); larger
 // tensors stay with the others too.
 bool f32_split_walk(const AttnParams& p, int D, int heads, bool backward) {
